@@ -279,6 +279,19 @@ __device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, int32x4_t rsr
                  : "memory", "m0");
 }
 
+// dma16 with a scalar offset added to every lane's. The range check may or may
+// not count it, so a lane's voff alone must decide what is out of range, and a
+// zero-length resource takes soff 0.
+__device__ __forceinline__ void dma16_at(uint32_t lds, uint32_t voff, int32x4_t rsrc, uint32_t soff) {
+    // uniform values that the compiler keeps in vector registers come back to scalar ones
+    const int32x4_t r = {__builtin_amdgcn_readfirstlane(rsrc[0]), __builtin_amdgcn_readfirstlane(rsrc[1]),
+                         __builtin_amdgcn_readfirstlane(rsrc[2]), 0x00020000};
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane(soff))
+                 : "memory", "m0");
+}
+
 // buffer_load_dword ... lds: lane l's 4 bytes at rsrc + voff land at LDS
 // lds + 4 * l (same contract as dma16).
 __device__ __forceinline__ void dma4(uint32_t lds, uint32_t voff, int32x4_t rsrc) {

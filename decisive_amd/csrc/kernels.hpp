@@ -72,6 +72,13 @@ void launch_w4a16(const Weight &w, const half_t *x, int m, float *y, int gemv_va
 // W4A16 with f16 output and optional fused epilogue (0 none, 1 GELU, 2 +residual f16)
 void launch_w4a16_f16(const Weight &w, const half_t *x, int m, half_t *y, int epilogue,
                       const half_t *residual, int variant, hipStream_t s);
+// W4A16 on the small deep-pipelined tiles (products_small.hip), tile an index
+// of its table; epi 0 f32 output, 1..3 f16 (plain, GELU, + residual). False
+// (nothing launched) where a block's panels pass 32-bit offsets.
+// w4a16_small_tile picks the tile by the grid, -1 where none pays.
+int w4a16_small_tile(int m, int n);
+bool launch_w4a16_small(const Weight &w, const half_t *x, int m, void *y, int epi, const half_t *res, int tile,
+                        hipStream_t s);
 // Per-row int8 GEMM: raw int32 or f32 epilogue. With b_q4, b is the per-row Q4
 // word buffer of launch_q4_quantize_rows (codes expanded to int8 in registers).
 void launch_i8_gemm(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb,

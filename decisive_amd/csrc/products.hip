@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "tiles.hpp"
 
 namespace dz {
 
@@ -1193,24 +1194,6 @@ __global__ __launch_bounds__(WM *WN * 64) void i8_gemm_kernel(const int8_t *__re
 }
 
 
-// Tiles are assigned XCD-aware: consecutive block ids go to different XCDs,
-// so tile ids are taken in XCD-major order and grouped GROUP_M tile-rows at a
-// time, keeping the blocks that share an XCD's L2 on neighbouring tiles.
-
-__device__ __forceinline__ void xcd_tile(int bid, int nblocks, int tiles_m, int tiles_n, int &tm, int &tn) {
-    constexpr int XCDS = 8, GROUP_M = 4;
-    int linear = bid;
-    if (nblocks % XCDS == 0) linear = (bid % XCDS) * (nblocks / XCDS) + bid / XCDS;
-    const int per_group = GROUP_M * tiles_n;
-    const int group = linear / per_group;
-    const int first_m = group * GROUP_M;
-    const int gsize = min(tiles_m - first_m, GROUP_M);
-    const int in_group = linear % per_group;
-    tm = first_m + in_group % gsize;
-    tn = in_group / gsize;
-}
-
-
 typedef int int16_t_v __attribute__((ext_vector_type(16)));
 
 // Deep-pipelined per-row int8 GEMM. Block tile BM x BN over 4 waves (2 x 2),
@@ -1653,21 +1636,6 @@ __global__ __launch_bounds__(WGM *WGN * 64, 2) void i8_gemm_stream_kernel(const 
 // pipelined W4A16 GEMM (large M)
 // ============================================================================
 
-// unpack_codes without asm: lo/hi masks come in SGPRs and the exponent in a
-// VGPR, so each (w & mask) | magic is one v_and_or_b32
-__device__ __forceinline__ uint4_t unpack_codes_c(uint32_t w, uint32_t mlo, uint32_t mhi, uint32_t magic) {
-    const half2_t bias = {(half_t)-1032.0f, (half_t)-1032.0f};
-    const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
-    const half2_t bias16 = {(half_t)-72.0f, (half_t)-72.0f};
-    const uint32_t w8 = w >> 8;
-    uint4_t out;
-    out[0] = half2_as_word(word_as_half2((w & mlo) | magic) + bias);
-    out[1] = half2_as_word(__builtin_elementwise_fma(word_as_half2((w & mhi) | magic), sixteenth, bias16));
-    out[2] = half2_as_word(word_as_half2((w8 & mlo) | magic) + bias);
-    out[3] = half2_as_word(__builtin_elementwise_fma(word_as_half2((w8 & mhi) | magic), sixteenth, bias16));
-    return out;
-}
-
 // Block tile BM x BN over WGM x WGN waves; one k-step is one 128-k block, in
 // two LDS stages filled by buffer_load ... lds while the other is computed:
 //  - activations: BM rows of 256 bytes; chunk c (8 halves) of row r sits at
@@ -1679,7 +1647,9 @@ __device__ __forceinline__ uint4_t unpack_codes_c(uint32_t w, uint32_t mlo, uint
 //  - scale records go straight to registers, one step ahead.
 // The stage loads are issued as asm (dma16) and waited for at the step's
 // barrier; the one compute body reads whichever stage is current. Needs
-// k % 128 == 0 (the launcher falls back otherwise).
+// k % 128 == 0, or RAGGED (k % 8 == 0): the chunks of a partial last block,
+// which hold the next row's values, are then cleared in LDS before that step
+// (a form of its own: the test for it costs config 5's product 0.5%).
 // Codes become f16 exactly as in gemm_w4a16_kernel (exact code times the f16
 // scale, rounded once), and each output accumulates one
 // v_mfma_f32_16x16x32_f16 per 32-k run in k order, so both kernels give the
@@ -1693,7 +1663,8 @@ __device__ __forceinline__ uint4_t unpack_codes_c(uint32_t w, uint32_t mlo, uint
 // block per tile) as one stream of k-steps: the last step of a tile loads the
 // next tile's first stage, so those loads fly during the epilogue. Each
 // tile's arithmetic is unchanged, so both forms give the same bits.
-template <int BM, int BN, int WGM, int WGN, bool G32, int EPI, int VALU_PER_MFMA = 2, bool PERSIST = false>
+template <int BM, int BN, int WGM, int WGN, bool G32, int EPI, int VALU_PER_MFMA = 2, bool PERSIST = false,
+          bool RAGGED = false>
 __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_pipe_kernel(
     const uint8_t *__restrict__ codes, const uint8_t *__restrict__ scales, const half_t *__restrict__ x, int m,
     int k, int n, int kbs, void *__restrict__ out, const half_t *__restrict__ residual, int ldo) {
@@ -1748,7 +1719,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_pipe_kernel(
     constexpr int DMA_GROUPS = 2;
     constexpr int DMA_N = XPW + WPW;
     // loads [DMA_N*part/DMA_GROUPS, DMA_N*(part+1)/DMA_GROUPS) of one stage
-    // (k % 128 == 0: every chunk of a step is inside the row)
+    // (RAGGED: chunks past k load the next row's values; past the last row, zeros)
     auto dma_part = [&](int stage, int kb, int part, int32x4_t rx, int32x4_t rw) {
         const int kk = kb * 128;
 #pragma unroll
@@ -1864,6 +1835,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_pipe_kernel(
             // (and every wave has finished reading the stage the next loads overwrite)
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0); the compiler sees it too
             __builtin_amdgcn_s_barrier();
+            if (RAGGED && kb + 1 == kbs) {  // the chunks past k hold the next row's values
+                const int ktail = k & 127;
+                for (int i = threadIdx.x; i < BM * 16; i += WAVES * 64)
+                    if ((i & 15) * 8 >= ktail)
+                        *(uint4_t *)(xs + stage * XSTAGE + i / 16 * 256 + ((i ^ (i >> 4)) & 15) * 16) = uint4_t{0, 0, 0, 0};
+                __syncthreads();
+            }
             const bool more = kb + 1 < kbs;
             if (more) load_scales(nsc, kb + 1, cur_t.srec);
             else if (has_next) load_scales(nsc, 0, nxt_t.srec);
@@ -1885,44 +1863,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_pipe_kernel(
             for (int nt = 0; nt < NT; nt++) {
                 const int c = col0 + wn * TN + nt * 16 + 4 * q;
                 if (c >= n) continue;
-                const size_t at = (size_t)r * ldo + c;
-                float v[4] = {acc[mb][nt][0], acc[mb][nt][1], acc[mb][nt][2], acc[mb][nt][3]};
-                if (EPI == 0) {
-                    if (vec) {
-                        *(float4_t *)((float *)out + at) = float4_t{v[0], v[1], v[2], v[3]};
-                    } else {
-                        for (int e = 0; e < 4; e++)
-                            if (c + e < n) ((float *)out)[at + e] = v[e];
-                    }
-                } else {
-                    half_t o[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        if (EPI == 1) o[e] = (half_t)v[e];
-                        else if (EPI == 2) o[e] = (half_t)f32_rounded(gelu_erf(v[e]));
-                        else o[e] = (half_t)0.0f;
-                    }
-                    if (EPI == 3) {
-                        if (vec) {
-                            const uint2_t rw = *(const uint2_t *)(residual + at);
-                            const half2_t r01 = word_as_half2(rw[0]), r23 = word_as_half2(rw[1]);
-                            o[0] = (half_t)f32_rounded(v[0] + (float)r01[0]);
-                            o[1] = (half_t)f32_rounded(v[1] + (float)r01[1]);
-                            o[2] = (half_t)f32_rounded(v[2] + (float)r23[0]);
-                            o[3] = (half_t)f32_rounded(v[3] + (float)r23[1]);
-                        } else {
-                            for (int e = 0; e < 4; e++)
-                                if (c + e < n) o[e] = (half_t)f32_rounded(v[e] + (float)residual[at + e]);
-                        }
-                    }
-                    if (vec) {
-                        const half2_t o01 = {o[0], o[1]}, o23 = {o[2], o[3]};
-                        *(uint2_t *)((half_t *)out + at) = uint2_t{half2_as_word(o01), half2_as_word(o23)};
-                    } else {
-                        for (int e = 0; e < 4; e++)
-                            if (c + e < n) ((half_t *)out)[at + e] = o[e];
-                    }
-                }
+                w4a16_store<EPI>(acc[mb][nt], out, residual, (size_t)r * ldo + c, c, n, vec);
             }
         }
         if (!has_next) break;
@@ -2472,14 +2413,13 @@ __global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
     }
 }
 
-inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
-
 // ---- variant tables -------------------------------------------------------------
 
 const char *const kGemvNames[] = {"auto", "w16", "w8", "stream8", "stream4", "persist"};
 const char *const kGemmNames[] = {"pipe-auto",   "256x256p2w8", "128x128p2w4", "128x256p2w8",
                                    "256x128w2x2", "128x128w2x2", "128x64w2x2", "256x256p2w8-persist",
-                                   "256x192p2w8-persist", "256x128p2w8"};
+                                   "256x192p2w8-persist", "256x128p2w8", "small32x32",
+                                   "small32x64", "small64x64", "small64x128"};
 const char *const kI8Names[] = {"256x256p2w8", "256x256p4k64w8", "256x128p3w8", "256x128p3",
                                  "128x128w2x2", "256x128w2x2", "64x64w2x2", "256x256p2w8-stream",
                                  "256x256p2w8-stream-mid", "256x128k64p2-stream2"};
@@ -2624,8 +2564,8 @@ template <int BM, int BN, int WGM, int WGN, int EPI, bool PERSIST = false>
 bool w4a16_pipe_launch(const Weight &w, const half_t *x, int m, void *y, const half_t *res, hipStream_t s,
                        int c0 = 0, int nc = -1) {
     if (nc < 0) nc = w.rows - c0;
-    // whole 128-k steps; byte offsets are 32-bit and relative to the block's first row / tile
-    if (w.cols % 128 != 0 || c0 % 16 != 0 || (size_t)BM * w.cols * 2 >= ((size_t)1 << 31) ||
+    // byte offsets are 32-bit and relative to the block's first row / tile
+    if (c0 % 16 != 0 || (size_t)BM * w.cols * 2 >= ((size_t)1 << 31) ||
         (size_t)(BN / 16) * w.kblocks() * 1024 >= ((size_t)1 << 31))
         return false;
     if (nc <= 0) return true;
@@ -2637,6 +2577,20 @@ bool w4a16_pipe_launch(const Weight &w, const half_t *x, int m, void *y, const h
     const unsigned tiles = cdiv(m, BM) * cdiv(nc, BN);
     // persistent: one block per compute unit (a multiple of the 8 XCDs), each taking every gridDim-th tile
     const unsigned blocks = PERSIST ? std::min(tiles, (unsigned)device_cus() / 8 * 8) : tiles;
+    if (w.cols % 128 != 0) {
+        if constexpr (BM == BN && !PERSIST) {
+            if (w.kind == WeightKind::Q4G32)
+                hipLaunchKernelGGL((w4a16_pipe_kernel<BM, BN, WGM, WGN, true, EPI, 2, false, true>), dim3(blocks),
+                                   dim3(WGM * WGN * 64), 0, s, codes, scales, x, m, w.cols, nc, w.kblocks(), yo, ro,
+                                   w.rows);
+            else
+                hipLaunchKernelGGL((w4a16_pipe_kernel<BM, BN, WGM, WGN, false, EPI, 2, false, true>), dim3(blocks),
+                                   dim3(WGM * WGN * 64), 0, s, codes, scales, x, m, w.cols, nc, w.kblocks(), yo, ro,
+                                   w.rows);
+            return true;
+        }
+        return false;
+    }
     if (w.kind == WeightKind::Q4G32)
         hipLaunchKernelGGL((w4a16_pipe_kernel<BM, BN, WGM, WGN, true, EPI, 2, PERSIST>), dim3(blocks),
                            dim3(WGM * WGN * 64), 0, s, codes, scales, x, m, w.cols, nc, w.kblocks(), yo, ro, w.rows);
@@ -2650,22 +2604,33 @@ bool w4a16_pipe_launch(const Weight &w, const half_t *x, int m, void *y, const h
 
 // Variants 0-3 are the pipelined kernel: "auto", 256x256 tiles on 8 waves
 // (one block per CU), 128x128 tiles on 4 waves (two blocks per CU) and
-// 128x256 tiles on 8 waves. "auto" runs persistent 256x256 tiles when they
+// 128x256 tiles on 8 waves; 10-13 the small tiles of products_small.hip.
+// "auto" runs a small tile where its grid fits one wave of compute units
+// (w4a16_small_tile), else persistent 256x256 tiles when they
 // fill two or more whole waves of compute units, else persistent 256x192
 // tiles when those do, else 256x256 tiles over the leading
 // columns that fill whole waves of compute units and 128x256 tiles over the
 // rest (one launch each), or, below one wave of 256x256 tiles, the largest of
 // 256x128, 128x256 and 128x128 that gives at least one tile per unit. 4-6 stage
 // through registers. All give the same bits (same f16 dequantization, one MFMA per
-// 32-k run in k order); the pipelined ones need k % 128 == 0 and fall back to
-// 256x128w2x2 otherwise.
+// 32-k run in k order). Where k % 128 != 0 the pipelined kernel has 256x256
+// and 128x128 tiles; its other forms, and panels past 32-bit offsets, fall back
+// to 256x128w2x2 (K=1688, N=1063: 45 us at 1024 rows and 47 at 2048).
 template <int EPI>
 void gemm_dispatch(const Weight &w, const half_t *x, int m, void *y, const half_t *res, int variant,
                    hipStream_t s) {
+    const int small = variant == 0 ? w4a16_small_tile(m, w.rows) : variant - 10;
+    if (small >= 0 && launch_w4a16_small(w, x, m, y, EPI, res, small, s)) return;
     switch (variant) {
         case 0: {
             const unsigned cus = (unsigned)device_cus();
             const unsigned tm = cdiv(m, 256), tn = cdiv(w.rows, 256);
+            if (w.cols % 128 != 0) {  // the ragged form: 256x256 tiles from one per unit, else 128x128
+                if (tm * tn >= cus ? w4a16_pipe_launch<256, 256, 2, 4, EPI>(w, x, m, y, res, s)
+                                   : w4a16_pipe_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s))
+                    return;
+                break;
+            }
             const unsigned t192 = w.rows % 192 == 0 ? tm * (unsigned)(w.rows / 192) : 0;
             if (tm * tn >= 2 * cus && (tm * tn) % cus == 0) {
                 // whole waves of 256x256 tiles, two or more: one persistent block per compute unit
@@ -2747,7 +2712,7 @@ void gv_launch(const Weight &w, const void *a, const float *sa, int m, int abits
 int variant_count(const char *family) {
     std::string f(family);
     if (f == "gemv") return 6;
-    if (f == "gemm_w4a16") return 10;
+    if (f == "gemm_w4a16") return 14;
     if (f == "i8_gemm") return 10;
     if (f == "grouped") return 14;
     if (f == "mlp") return 6;

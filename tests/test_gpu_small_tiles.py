@@ -1,0 +1,74 @@
+"""The small-tile product kernels and the rules that choose them, against the
+kernels whose place they take: bit for bit."""
+import numpy as np
+import pytest
+
+from decisive_amd import rocm
+from gpu_util import bits_equal, dev, empty, host
+
+pytestmark = pytest.mark.gpu
+
+SMALL_W4A16 = ("small32x32", "small32x64", "small64x64", "small64x128", "pipe-auto")
+
+
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("m,k,n", [
+    (17, 8, 1), (33, 120, 63), (31, 128, 64), (32, 136, 65), (65, 256, 129),  # edges of tiles, one partial or whole block
+    (64, 384, 128), (63, 640, 127), (129, 1000, 272),                          # fewer steps than the ring, ragged k
+    (40, 4096, 4096), (200, 2568, 1040), (2100, 1688, 1063),                   # long rings; the ragged pipelined tiles
+])
+def test_w4a16_small_tiles_give_the_staged_kernels_bits(ctx, group, m, k, n):
+    """Every small tile and the automatic choice against the register-staged
+    kernel (pinned to the closed form elsewhere): the same MFMA per 32-k run in
+    k order, so the same bits, in f32 and through each f16 epilogue."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(m + k + n + group)
+    x = dev(rng.standard_normal((m, k)).astype(np.float16))
+    w = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.02).astype(np.float32)), rocm.F32, n, k, 4, group)
+    res = dev(rng.standard_normal((m, n)).astype(np.float16))
+
+    def outputs(name):
+        ctx.select_variant("gemm_w4a16", name)
+        y = empty((m, n), torch.float32)
+        ctx.linear(w, x, rocm.F16, m, y, rocm.W4A16)
+        outs = [host(ctx, y)]
+        for epi in (rocm.EPI_NONE, rocm.EPI_GELU, rocm.EPI_RESIDUAL):
+            h = empty((m, n), torch.float16)
+            ctx.linear_f16(w, x, m, h, epi, res if epi == rocm.EPI_RESIDUAL else None)
+            outs.append(host(ctx, h).view(np.uint16))
+        return outs
+
+    try:
+        want = outputs("256x128w2x2")
+        assert np.isfinite(want[0]).all()
+        for name in SMALL_W4A16:
+            got = outputs(name)
+            assert bits_equal(got[0], want[0]), name
+            assert all(np.array_equal(a, b) for a, b in zip(got[1:], want[1:])), name
+    finally:
+        ctx.select_variant("gemm_w4a16", "pipe-auto")
+
+
+@pytest.mark.parametrize("k", [1000, 4096])
+def test_w4a16_rows_do_not_see_each_other(ctx, k):
+    """A row of infinities beside finite ones: the chunks a partial block loads
+    past a row's end are the next row's and must not reach it."""
+    torch = pytest.importorskip("torch")
+    m, n = 70, 96
+    rng = np.random.default_rng(k)
+    clean = rng.standard_normal((m, k)).astype(np.float16)
+    dirty = clean.copy()
+    dirty[1::2] = np.inf
+    w = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.02).astype(np.float32)), rocm.F32, n, k, 4, 32)
+    try:
+        for name in SMALL_W4A16 + ("128x128p2w4", "256x256p2w8-persist"):
+            ctx.select_variant("gemm_w4a16", name)
+            outs = []
+            for v in (clean, dirty):
+                y = empty((m, n), torch.float32)
+                ctx.linear(w, dev(v), rocm.F16, m, y, rocm.W4A16)
+                outs.append(host(ctx, y))
+            assert bits_equal(outs[1][0::2], outs[0][0::2]), name
+            assert not np.isfinite(outs[1][1::2]).any(), name
+    finally:
+        ctx.select_variant("gemm_w4a16", "pipe-auto")
