@@ -83,6 +83,10 @@ bool launch_w4a16_small(const Weight &w, const half_t *x, int m, void *y, int ep
 // word buffer of launch_q4_quantize_rows (codes expanded to int8 in registers).
 void launch_i8_gemm(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb,
                     int n, int k, void *y, int raw, int variant, hipStream_t s, bool b_q4 = false);
+// The same product for a few rows (products_small.hip), streaming the weight;
+// false (nothing launched) where k or the operands are not whole words.
+bool launch_i8_rows(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k, void *y,
+                    int raw, hipStream_t s);
 // webgpu/int8.rs:226-230 gemm(fused=true): y = silu(gate) * up of two per-row int8 products sharing a
 void launch_i8_gemm_fused(const int8_t *a, const float *sa, int m, const int8_t *wg, const float *sg,
                           const int8_t *wu, const float *su, int n, int k, float *y, hipStream_t s);

