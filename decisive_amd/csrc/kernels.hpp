@@ -133,7 +133,7 @@ int device_cus();
 // 16 or 32 state columns per block; ws holds delta_chunk_ws_bytes).
 void launch_delta_scan_tokens(const float *qhat, const float *khat, const float *conv, const float *gb, int n,
                               int lh, int lk, float *out, bool rolled, hipStream_t s);
-size_t delta_chunk_ws_bytes(int n, int lh);
+size_t delta_chunk_ws_bytes(int n, int lh, int lk);
 void launch_delta_scan_chunked(const float *qhat, const float *khat, const float *conv, const float *gb, int n,
                                int lh, int lk, float *ws, float *out, int column_tiles, hipStream_t s);
 

@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <string>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "../../include/decisive_rocm.h"
@@ -283,21 +284,56 @@ __global__ __launch_bounds__(kScanWaves * 64) void delta_scan_kernel(const float
 // order for 16 state columns per block.
 constexpr int kChunk = 64;
 constexpr int kChunkWs = 2 * kChunk * kLd + kChunk * kChunk + kLd * kChunk + kChunk;  // floats per (head, chunk)
-constexpr int kChunkRow = kLd + 4;    // padded LDS row of K / Q (conflict-free float4 reads across rows)
+constexpr int kChunkQ = kChunk * kLd;  // floats of a (key head, chunk)'s Q record
+constexpr int kChunkRow = kLd + 4;    // padded LDS row of K (conflict-free float4 reads across rows)
+constexpr int kTriRow = kChunk + 4;   // the same for P
 
-// One block (4 waves) per (head, chunk). Workspace record (floats):
-// Uv [64][128] | Wk [64][128] | P [64][64] | rKT [128][64] (gamma_last/gamma_t K[t][dk]) | gamma [64].
+// One block (4 waves) per (head, chunk). The workspace record is written in
+// the order the scan's lanes read it, so that each of its loads is one
+// contiguous KiB (lane (col, g) of wave w, 16 bytes each; when a load touched
+// 64 cache lines the scan took 81 us at 1024 tokens, now 57):
+//   Uv  [8 column blocks y][w][lane]: rows 16w + 4g + 0..3 of column 16y + col
+//   Wk  [w][i < 8][lane]:             row 16w + col, dims 32g + 4i + 0..3
+//   P   [w][i < 4][lane]:             row 16w + col, tokens 16g + 4i + 0..3
+//   rKT [w][d < 2][i < 4][lane]:      dim 32w + 16d + col, tokens 16g + 4i + 0..3
+//                                     (gamma_last / gamma_t K[t][dim])
+//   gamma [64]
+// then, after every head's records, a Q record per (key head, chunk) in Wk's order.
+//
+// The triangular system is solved row by row, one right-hand side per thread,
+// in a loop over 16-row blocks whose code is reused: unrolled over all 64 rows
+// it was 16 KB of instructions that each wave fetched once, and their fetch
+// bounded the kernel (53.6 us at 1024 tokens and 40.3 at 229, one block per unit
+// at most, now 40.5 and 27.9; DPP alone, unrolled: 50.6 and 39.5). The row
+// of A that a step needs is the same for every thread: 16 values of it sit in
+// the lanes of each 16-lane row of a register, and v_fmac_f32 takes one of them
+// by DPP row broadcast. Solved columns go to LDS (over K, and beside it for V).
+template <class F, int... I>
+__device__ __forceinline__ void each_index(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+// acc = fma(lane L of a's 16-lane row, x, acc). As asm, since the compiler leaves
+// the broadcast a move of its own; the operand `a` comes from LDS and passes
+// dpp_ready first (a DPP read needs two wait states after a VALU write).
+template <int L>
+__device__ __forceinline__ float fma_row_lane(float a, float x, float acc) {
+    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(a), "v"(x), "n"(L));
+    return acc;
+}
+__device__ __forceinline__ void dpp_ready(float &a) { asm volatile("s_nop 1" : "+v"(a)); }
+
 __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__restrict__ qhat,
                                                                const float *__restrict__ khat,
                                                                const float *__restrict__ conv,
                                                                const float *__restrict__ gb, int n, int lh, int lk,
                                                                float *__restrict__ ws) {
     extern __shared__ __align__(16) float sm[];
-    float *ks = sm, *as = ks + kChunk * kChunkRow, *cum = as + kChunk * kChunk, *bet = cum + kChunk,
-          *bk = bet + kChunk;
+    float *ks = sm, *vs = ks + kChunk * kChunkRow, *as = vs + kChunk * kChunkRow, *cum = as + 10 * 256,
+          *bet = cum + kChunk, *bk = bet + kChunk, *rel = bk + kChunk;
+    float *ps = vs;  // P, until it has left for the record
     const int h = blockIdx.x, c = blockIdx.y, tid = threadIdx.x;
-    const int wave = tid / 64, lane = tid % 64, col = lane % 16, g = lane / 16;
-    const int kh = h / (lh / lk), t0 = c * kChunk;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64, col = lane % 16, g = lane / 16;
+    const int per = lh / lk, kh = h / per, t0 = c * kChunk;
     const size_t lkv = (size_t)lk * kLd, width = 2 * lkv + (size_t)lh * kLd;
     float *rec = ws + ((size_t)h * gridDim.y + c) * kChunkWs;
     float *uv = rec, *wk = uv + kChunk * kLd, *pm = wk + kChunk * kLd, *rkt = pm + kChunk * kChunk,
@@ -324,7 +360,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__re
         bet[tid] = tok < n ? gb[((size_t)tok * lh + h) * 4 + 1] : 0.0f;
         cum[tid] = tok < n ? gb[((size_t)tok * lh + h) * 4 + 3] : 0.0f;
     }
-    // this lane's Q fragment (row 16*wave + col, dims 32g..32g+31) for Q K^T
+    // this lane's Q fragment (row 16*wave + col, dims 32g..32g+31) for Q K^T and the scan
     float4_t qf[8];
     {
         const int tok = t0 + 16 * wave + col;
@@ -335,97 +371,165 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__re
     }
     __syncthreads();
     if (tid == 0) {  // the running sum of log g in token order, in registers (16-byte LDS reads and writes)
-        float4_t c[kChunk / 4];
+        float4_t v[kChunk / 4];
 #pragma unroll
-        for (int i = 0; i < kChunk / 4; i++) c[i] = *(const float4_t *)(cum + 4 * i);
+        for (int i = 0; i < kChunk / 4; i++) v[i] = *(const float4_t *)(cum + 4 * i);
         float run = 0.0f;
 #pragma unroll
         for (int i = 0; i < kChunk / 4; i++)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                run += c[i][e];
-                c[i][e] = run;
+                run += v[i][e];
+                v[i][e] = run;
             }
 #pragma unroll
-        for (int i = 0; i < kChunk / 4; i++) *(float4_t *)(cum + 4 * i) = c[i];
+        for (int i = 0; i < kChunk / 4; i++) *(float4_t *)(cum + 4 * i) = v[i];
     }
     __syncthreads();
-    if (tid < kChunk) bk[tid] = bet[tid] * expf(cum[tid]);
-    // K K^T and Q K^T, row block `wave`: lane (col, g) holds rows 16*wave + 4g + i of column block cb
-#pragma unroll 1
-    for (int cb = 0; cb < 4; cb++) {
-        float4_t kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
-        const float *ka = ks + (16 * wave + col) * kChunkRow + 32 * g;
+    if (tid < kChunk) {
+        const float gamma = expf(cum[tid]);
+        bk[tid] = bet[tid] * gamma;
+        rel[tid] = expf(cum[kChunk - 1] - cum[tid]);
+        gam[tid] = gamma;
+    }
+    // Q K^T for row block `wave` and K K^T for row block 3 - wave: with the
+    // column blocks past the diagonal left out, five 16x16x128 products a wave
+    auto tile = [&](const float4_t *a, int cb) {  // A rows x K rows 16 cb ..
         const float *kb = ks + (16 * cb + col) * kChunkRow + 32 * g;
+        float4_t d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            const float4_t a4 = *(const float4_t *)(ka + 4 * i), b4 = *(const float4_t *)(kb + 4 * i);
+            const float4_t b4 = *(const float4_t *)(kb + 4 * i);
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                kk = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[e], b4[e], kk, 0, 0, 0);
-                qk = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[i][e], b4[e], qk, 0, 0, 0);
-            }
+            for (int e = 0; e < 4; e++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b4[e], d, 0, 0, 0);
         }
+        return d;
+    };
+#pragma unroll 1
+    for (int cb = 0; cb < 4; cb++) {
+        const float4_t qk = cb <= wave ? tile(qf, cb) : float4_t{0.f, 0.f, 0.f, 0.f};
         const int j = 16 * cb + col;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int r = 16 * wave + 4 * g + i;
-            const float d = j <= r ? expf(cum[r] - cum[j]) : 0.0f;
-            as[r * kChunk + j] = j < r ? bet[r] * d * kk[i] : 0.0f;
-            pm[r * kChunk + j] = d * qk[i];
+            ps[r * kTriRow + j] = j <= r ? expf(cum[r] - cum[j]) * qk[i] : 0.0f;
+        }
+    }
+    if (h % per == 0) {
+        float *qrec = ws + (size_t)lh * gridDim.y * kChunkWs + ((size_t)kh * gridDim.y + c) * kChunkQ;
+#pragma unroll
+        for (int i = 0; i < 8; i++) *(float4_t *)(qrec + ((wave * 8 + i) * 64 + lane) * 4) = qf[i];
+    }
+    {
+        const int rb = 3 - wave;
+        float4_t kf[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) kf[i] = *(const float4_t *)(ks + (16 * rb + col) * kChunkRow + 32 * g + 4 * i);
+#pragma unroll 1
+        for (int cb = 0; cb <= rb; cb++) {
+            const float4_t kk = tile(kf, cb);
+            const int j = 16 * cb + col;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int r = 16 * rb + 4 * g + i;
+                as[(rb * (rb + 1) / 2 + cb) * 256 + (4 * g + i) * 16 + col] = j < r ? bet[r] * expf(cum[r] - cum[j]) * kk[i] : 0.0f;
+            }
         }
     }
     __syncthreads();
-    // (I + A) x = b, one right-hand side per thread: columns of diag(beta) V
-    // (waves 0-1), then of diag(beta gamma) K (waves 2-3)
-    auto solve = [&](auto vcol_c) {
-        constexpr bool VCOL = decltype(vcol_c)::value;
-        const int cc = VCOL ? tid : tid - kLd;
-        const float *vsrc = conv + 2 * lkv + (size_t)h * kLd + cc;
-        float x[kChunk];  // the right-hand side, then the solution in place
+    // (gamma_last / gamma_t) K[t][dim] in the scan's order
 #pragma unroll
-        for (int i = 0; i < kChunk; i++) {
-            if (VCOL) x[i] = t0 + i < n ? bet[i] * vsrc[(size_t)(t0 + i) * width] : 0.0f;
-            else x[i] = bk[i] * ks[i * kChunkRow + cc];
-        }
-        __builtin_amdgcn_sched_barrier(0);
+    for (int d = 0; d < 2; d++)
 #pragma unroll
-        for (int i = 1; i < kChunk; i++) {
-            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-#pragma unroll
-            for (int l = 0; l + 3 < i; l += 4) {
-                const float4_t a4 = *(const float4_t *)(as + i * kChunk + l);
-                s0 = __builtin_fmaf(a4[0], x[l], s0);
-                s1 = __builtin_fmaf(a4[1], x[l + 1], s1);
-                s2 = __builtin_fmaf(a4[2], x[l + 2], s2);
-                s3 = __builtin_fmaf(a4[3], x[l + 3], s3);
-            }
-#pragma unroll
-            for (int l = i & ~3; l < i; l++) s0 = __builtin_fmaf(as[i * kChunk + l], x[l], s0);
-            x[i] -= (s0 + s1) + (s2 + s3);
-        }
-        float *dst = VCOL ? uv : wk;
-#pragma unroll
-        for (int i = 0; i < kChunk; i++) dst[i * kLd + cc] = x[i];
-    };
-    if (__builtin_amdgcn_readfirstlane(wave) < 2) solve(std::true_type{});
-    else solve(std::false_type{});
-    // (gamma_last / gamma_t) K[t][dk], transposed; gamma_t
-    {
-        const int dk = tid / 2, th = (tid % 2) * 32;
-        const float last = cum[kChunk - 1];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int i = 0; i < 4; i++) {
             float4_t v4;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int t = th + 4 * u + e;
-                v4[e] = expf(last - cum[t]) * ks[t * kChunkRow + dk];
+                const int t = 16 * g + 4 * i + e;
+                v4[e] = rel[t] * ks[t * kChunkRow + 32 * wave + 16 * d + col];
             }
-            *(float4_t *)(rkt + dk * kChunk + th + 4 * u) = v4;
+            *(float4_t *)(rkt + (((wave * 2 + d) * 4 + i) * 64 + lane) * 4) = v4;
         }
-        if (tid < kChunk) gam[tid] = expf(cum[tid]);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        *(float4_t *)(pm + ((wave * 4 + i) * 64 + lane) * 4) =
+            *(const float4_t *)(ps + (16 * wave + col) * kTriRow + 16 * g + 4 * i);
+    // (I + A) x = b, one right-hand side per thread: columns of diag(beta) V
+    // (waves 0-1), then of diag(beta gamma) K (waves 2-3). Row i takes its sum in
+    // four parts (l % 4) over the whole quads below the diagonal, then the rest
+    // onto the first.
+    const bool vcol = wave < 2;
+    const int cc = vcol ? tid : tid - kLd;
+    float *const xcol = (vcol ? vs : ks) + cc;  // this column, solved rows in place
+    const float *const vsrc = conv + 2 * lkv + (size_t)h * kLd + cc;
+    float nx[16];  // the next block's right-hand side, its loads in flight over a block
+    auto fetch_rhs = [&](int b) {
+        if (vcol) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int i = 16 * b + r;
+                nx[r] = t0 + i < n ? vsrc[(size_t)(t0 + i) * width] : 0.0f;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; r++) nx[r] = xcol[(16 * b + r) * kChunkRow];
+        }
+    };
+    fetch_rhs(0);
+    __syncthreads();  // the last reads of P and of K by other threads are done
+#pragma unroll 1
+    for (int b = 0; b < 4; b++) {
+        float x[16], s[16][4];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int i = 16 * b + r;
+            x[r] = vcol ? (t0 + i < n ? bet[i] * nx[r] : 0.0f) : bk[i] * nx[r];
+#pragma unroll
+            for (int e = 0; e < 4; e++) s[r][e] = 0.0f;
+        }
+        if (b < 3) fetch_rhs(b + 1);
+        const float *ab = as + b * (b + 1) / 2 * 256 + col;
+#pragma unroll 1
+        for (int c = 0; c < b; c++, ab += 256) {  // rows of block b against the solved block c
+            float xc[16];
+#pragma unroll
+            for (int l = 0; l < 16; l++) xc[l] = xcol[(16 * c + l) * kChunkRow];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                float a = ab[r * 16];
+                dpp_ready(a);
+                each_index([&](auto l) { s[r][l % 4] = fma_row_lane<l>(a, xc[l], s[r][l % 4]); },
+                           std::make_integer_sequence<int, 16>{});
+            }
+        }
+        each_index(
+            [&](auto row) {
+                constexpr int r = decltype(row)::value;
+                float a = ab[r * 16];
+                dpp_ready(a);
+                each_index(
+                    [&](auto l) {
+                        constexpr int part = l < (r & ~3) ? l % 4 : 0;
+                        if constexpr (l < r) s[r][part] = fma_row_lane<l>(a, x[l], s[r][part]);
+                    },
+                    std::make_integer_sequence<int, 16>{});
+                if (r > 0 || b > 0) x[r] -= (s[r][0] + s[r][1]) + (s[r][2] + s[r][3]);
+            },
+            std::make_integer_sequence<int, 16>{});
+#pragma unroll
+        for (int r = 0; r < 16; r++) xcol[(16 * b + r) * kChunkRow] = x[r];
+        if (vcol) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *(float4_t *)(uv + ((cc / 16 * 4 + b) * 64 + q * 16 + cc % 16) * 4) =
+                    float4_t{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+        }
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        *(float4_t *)(wk + ((wave * 8 + i) * 64 + lane) * 4) =
+            *(const float4_t *)(ks + (16 * wave + col) * kChunkRow + 32 * g + 4 * i);
 }
 
 // One block per (head, CT x 16 state columns), 4 waves per 16 columns; the
@@ -435,8 +539,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__re
 // state column's arithmetic is the same for every CT, so CT = 1 and CT = 2
 // give the same bits (CT = 2: half the blocks, eight waves each).
 template <int CT>
-__global__ __launch_bounds__(256 * CT) void delta_chunk_scan_kernel(const float *__restrict__ qhat,
-                                                                    const float *__restrict__ ws, int n, int lh,
+__global__ __launch_bounds__(256 * CT) void delta_chunk_scan_kernel(const float *__restrict__ ws, int n, int lh,
                                                                     int lk, float *__restrict__ out) {
     constexpr int UROW = kChunk + 4;
     __shared__ __align__(16) float st_all[CT * 16 * kChunkRow];  // S_T [16][128 + 4] per column tile
@@ -452,29 +555,27 @@ __global__ __launch_bounds__(256 * CT) void delta_chunk_scan_kernel(const float 
     // the global operands of one chunk for this lane; the next chunk's are in
     // flight while the current one computes
     struct Ops {
-        float4_t w[8], q[8], p[4], r[2][4];
-        float u[4], gm[4], last;
+        float4_t w[8], q[8], p[4], r[2][4], u, gm;
+        float last;
     };
     auto fetch = [&](int c) {
         Ops o;
         const float *rec = ws + ((size_t)h * chunks + c) * kChunkWs;
         const float *uv = rec, *wk = uv + kChunk * kLd, *pm = wk + kChunk * kLd, *rkt = pm + kChunk * kChunk,
                     *gam = rkt + kLd * kChunk;
-        const int row = 16 * wave + col, tq = min(c * kChunk + row, n - 1);
-        const float *qa = qhat + ((size_t)tq * lk + kh) * kLd + 32 * g;
+        const float *qr = ws + (size_t)lh * chunks * kChunkWs + ((size_t)kh * chunks + c) * kChunkQ;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            o.w[i] = *(const float4_t *)(wk + row * kLd + 32 * g + 4 * i);
-            o.q[i] = *(const float4_t *)(qa + 4 * i);
+            o.w[i] = *(const float4_t *)(wk + ((wave * 8 + i) * 64 + lane) * 4);
+            o.q[i] = *(const float4_t *)(qr + ((wave * 8 + i) * 64 + lane) * 4);
         }
+        o.u = *(const float4_t *)(uv + ((col0 / 16 * 4 + wave) * 64 + lane) * 4);
+        o.gm = *(const float4_t *)(gam + 16 * wave + 4 * g);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            o.p[i] = *(const float4_t *)(pm + row * kChunk + 16 * g + 4 * i);
+            o.p[i] = *(const float4_t *)(pm + ((wave * 4 + i) * 64 + lane) * 4);
 #pragma unroll
-            for (int d = 0; d < 2; d++) o.r[d][i] = *(const float4_t *)(rkt + (32 * wave + 16 * d + col) * kChunk + 16 * g + 4 * i);
-            const int t = 16 * wave + 4 * g + i;
-            o.u[i] = uv[t * kLd + col0 + col];
-            o.gm[i] = gam[t];
+            for (int d = 0; d < 2; d++) o.r[d][i] = *(const float4_t *)(rkt + (((wave * 2 + d) * 4 + i) * 64 + lane) * 4);
         }
         o.last = gam[kChunk - 1];
         return o;
@@ -843,12 +944,14 @@ void launch_delta_scan_tokens(const float *qhat, const float *khat, const float 
                            khat, conv, gb, n, lh, lk, out);
 }
 
-size_t delta_chunk_ws_bytes(int n, int lh) { return (size_t)lh * ((n + kChunk - 1) / kChunk) * kChunkWs * 4; }
+size_t delta_chunk_ws_bytes(int n, int lh, int lk) {
+    return ((size_t)lh * kChunkWs + (size_t)lk * kChunkQ) * ((n + kChunk - 1) / kChunk) * 4;
+}
 
 void launch_delta_scan_chunked(const float *qhat, const float *khat, const float *conv, const float *gb, int n,
                                int lh, int lk, float *ws, float *out, int column_tiles, hipStream_t s) {
     if (n <= 0) return;
-    constexpr size_t lds = (size_t)(kChunk * kChunkRow + kChunk * kChunk + 3 * kChunk) * 4;
+    constexpr size_t lds = (size_t)(2 * kChunk * kChunkRow + 10 * 256 + 4 * kChunk) * 4;
     static bool configured[64] = {};  // the LDS limit is a per-device function attribute
     int dev = 0;
     hipGetDevice(&dev);
@@ -861,9 +964,9 @@ void launch_delta_scan_chunked(const float *qhat, const float *khat, const float
     hipLaunchKernelGGL(delta_chunk_prep_kernel, dim3(lh, chunks), dim3(256), lds, s, qhat, khat, conv, gb, n, lh, lk,
                        ws);
     if (column_tiles == 2)
-        hipLaunchKernelGGL(delta_chunk_scan_kernel<2>, dim3(lh, kLd / 32), dim3(512), 0, s, qhat, ws, n, lh, lk, out);
+        hipLaunchKernelGGL(delta_chunk_scan_kernel<2>, dim3(lh, kLd / 32), dim3(512), 0, s, ws, n, lh, lk, out);
     else
-        hipLaunchKernelGGL(delta_chunk_scan_kernel<1>, dim3(lh, kLd / 16), dim3(256), 0, s, qhat, ws, n, lh, lk, out);
+        hipLaunchKernelGGL(delta_chunk_scan_kernel<1>, dim3(lh, kLd / 16), dim3(256), 0, s, ws, n, lh, lk, out);
 }
 
 }  // namespace dz
@@ -1002,7 +1105,7 @@ int32_t ensure_capacity(dz_ctx *ctx, dz_pplx *p, size_t n) {
     get(&p->qhat, n * c.delta_key_heads * kLd * 4);
     get(&p->khat, n * c.delta_key_heads * kLd * 4);
     get(&p->gb, n * c.delta_heads * 4 * 4);
-    get(&p->chunk_ws, delta_chunk_ws_bytes((int)n, c.delta_heads));
+    get(&p->chunk_ws, delta_chunk_ws_bytes((int)n, c.delta_heads, c.delta_key_heads));
     get(&p->heads, n * std::max(lv, (size_t)c.attn_heads * kAd) * 4);
     get(&p->ctx, n * ctxw * 4);
     get(&p->projected, n * d * 4);

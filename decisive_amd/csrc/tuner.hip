@@ -256,7 +256,7 @@ bool build_bench(DeviceBuffers &buf, const Family &f, int count, Bench *b) {
             b->khat = (const float *)buf.upload(hk);
             b->conv = (const float *)buf.upload(hc);
             b->gb = (const float *)buf.upload(hg);
-            b->chunk_ws = (float *)buf.alloc(delta_chunk_ws_bytes((int)M, (int)N));
+            b->chunk_ws = (float *)buf.alloc(delta_chunk_ws_bytes((int)M, (int)N, (int)K));
             break;
         }
         case Kind::Grouped:
