@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "ordered_sum.hpp"
 
 namespace dz {
 
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float *__restrict__ 
 // reference's iterator sum does, so the result is bit-exact with it. One
 // 256-thread block per selected row (`rows` picks hidden rows; null takes row
 // r): every thread squares its share of the row into LDS (loads in flight
-// together), thread 0 adds the squares in row order, and all threads write
+// together), wave 0 adds the squares in row order (ordered_sum), and all threads write
 // the scaled row.
 template <int DT>
 __global__ __launch_bounds__(256) void readout_rms_kernel(const void *__restrict__ h,
@@ -180,20 +181,9 @@ __global__ __launch_bounds__(256) void readout_rms_kernel(const void *__restrict
         squares[i] = __fmul_rn(v, v);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float ss = 0.0f;
-        int i = 0;
-        for (; i + 8 <= d; i += 8) {
-            const float4_t a = *(const float4_t *)(squares + i), b = *(const float4_t *)(squares + i + 4);
-            ss = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(ss, a[0]), a[1]), a[2]), a[3]);
-            ss = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(ss, b[0]), b[1]), b[2]), b[3]);
-        }
-        for (; i < d; i++) ss = __fadd_rn(ss, squares[i]);
-        // v_sqrt_f32 is not correctly rounded; a float's square root taken in
-        // f64 and rounded to f32 is (the exact root is never near enough to a
-        // float midpoint for the f64 error to matter)
-        const float t = __fadd_rn(__fdiv_rn(ss, (float)d), eps);
-        scale_sh = __fdiv_rn(1.0f, __double2float_rn(__dsqrt_rn((double)t)));
+    if (threadIdx.x < 64) {
+        const float ss = ordered_sum(squares, d);
+        if (threadIdx.x == 0) scale_sh = rms_row_scale(ss, d, eps);
     }
     __syncthreads();
     const float scale = scale_sh;

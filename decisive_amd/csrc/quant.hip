@@ -11,6 +11,7 @@
 #include <float.h>
 
 #include "kernels.hpp"
+#include "ordered_sum.hpp"
 
 namespace dz {
 
@@ -301,166 +302,82 @@ __global__ void act_quantize_kernel(const float *__restrict__ x, int m, int k, i
 
 // ---- zero-centred RMSNorm fused with the A8 quantizer -------------------------------
 //
-// Rows of d floats (d % 64 == 0), in two launches:
-//  1. rms_row_scale_kernel: lane l of wave 0 owns row 16 * block + l % 16
-//     and adds the row's squares in row order, as pplx_flash/cpu.rs:310-333
-//     does (the readout norm's arithmetic, bit for bit). Wave 1 streams
-//     64-column tiles of the block's 16 rows into 16 LDS stages by
-//     buffer_load ... lds, 14 tiles ahead, and squares each tile in place one
-//     tile ahead of wave 0, so wave 0's chain of d dependent adds is all it
-//     waits for. A tile row's 16-byte chunk c sits at slot c ^ row, so the 16
-//     rows' reads of one chunk index hit distinct banks. The row scale
-//     1 / sqrt(ss / d + eps) goes to sc[row * groups], the first of the row's
-//     group-scale slots.
-//  2. rms_apply_quantize_kernel: one block per row takes that scale, then every
-//     wave takes 64-column groups: v = (x * scale) * (1 + w) (w when not
-//     zero-centred), written to y when y is set, and the group's A8 codes and
-//     scale exactly as act_quantize_kernel computes them from v
-//     (int8.rs:178-202), so a product of these codes equals the product of y.
-//     A non-finite v sets *bad.
-constexpr int kRmsRows = 16;    // rows (chains) per block
-constexpr int kRmsStages = 16;  // 64-column tiles in LDS
-
-__global__ __launch_bounds__(128) void rms_row_scale_kernel(const float *__restrict__ h, int rows, int d, float eps,
-                                                            float *__restrict__ sc) {
-    __shared__ __align__(16) float stages[kRmsStages][kRmsRows * 64];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
-    const int row0 = blockIdx.x * kRmsRows;
-    const int nrows = min(kRmsRows, rows - row0), tiles = d / 64;
-    constexpr int PER_TILE = kRmsRows / 4;  // DMA instructions per tile
-    static_assert((kRmsStages - 2) * PER_TILE <= 63, "vmcnt range");
-    if (wave == 1) {
-        const int32x4_t rs = buffer_rsrc(h + (size_t)row0 * d, (uint32_t)(nrows * d * 4));
-        const uint32_t base = lds_address(&stages[0][0]);
-        // DMA instruction i of a tile fills rows 4i..4i+3: lane j -> row 4i + j / 16,
-        // slot j % 16, which holds the row's chunk (j % 16) ^ row
-        auto dma_tile = [&](int t) {
-            const int slot = t % kRmsStages;
-#pragma unroll
-            for (int i = 0; i < PER_TILE; i++) {
-                const int r = 4 * i + lane / 16, c = (lane % 16) ^ r;
-                dma16(base + (uint32_t)(slot * kRmsRows * 64 * 4 + i * 1024),
-                      (uint32_t)((r * d + t * 64 + 4 * c) * 4), rs);
-            }
-        };
-        auto square_tile = [&](int t) {
-            float4_t *p = (float4_t *)stages[t % kRmsStages];
-            float4_t v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = p[lane + 64 * i];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                p[lane + 64 * i] = float4_t{__fmul_rn(v[i][0], v[i][0]), __fmul_rn(v[i][1], v[i][1]),
-                                            __fmul_rn(v[i][2], v[i][2]), __fmul_rn(v[i][3], v[i][3])};
-        };
-#pragma unroll
-        for (int t = 0; t < kRmsStages - 1; t++)
-            if (t < tiles) dma_tile(t);
-        if (kRmsStages - 2 < tiles)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRmsStages - 2) * PER_TILE) : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        square_tile(0);
-        __syncthreads();
-        for (int t = 0; t < tiles; t++) {
-            if (t + 1 < tiles) {
-                // tile t + 1 landed (tiles up to t + NS - 2 are issued)
-                if (t + kRmsStages - 2 < tiles)
-                    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRmsStages - 3) * PER_TILE) : "memory");
-                else
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                square_tile(t + 1);
-                // wave 0 read tile t - 1 before the last barrier
-                if (t + kRmsStages - 1 < tiles) dma_tile(t + kRmsStages - 1);
-            }
-            __syncthreads();
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no LDS write in flight once the block ends
-        return;
-    }
-    const int r = lane % kRmsRows;
-    auto read_half = [&](int t, int half, float4_t *v) {
-        const float *row = &stages[t % kRmsStages][r * 64];
-#pragma unroll
-        for (int c = 0; c < 8; c++) v[c] = *(const float4_t *)(row + 4 * ((8 * half + c) ^ r));
-    };
-    float ss = 0.0f;
-    auto add_half = [&](const float4_t *v) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int c = 0; c < 8; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) ss = __fadd_rn(ss, v[c][e]);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    float4_t x0[8], x1[8];
-    __syncthreads();  // tile 0 squared
-    for (int t = 0; t < tiles; t++) {
-        read_half(t, 0, x0);
-        read_half(t, 1, x1);
-        add_half(x0);
-        add_half(x1);
-        __syncthreads();  // tile t read; tile t + 1 squared
-    }
-    if (lane < nrows) {
-        // the square root taken in f64 and rounded once (v_sqrt_f32 is not correctly rounded)
-        const float q = __fadd_rn(__fdiv_rn(ss, (float)d), eps);
-        sc[(size_t)(row0 + lane) * (d / 64)] = __fdiv_rn(1.0f, __double2float_rn(__dsqrt_rn((double)q)));
-    }
-}
-
-__global__ __launch_bounds__(256) void rms_apply_quantize_kernel(const float *__restrict__ h, int d,
-                                                                 const float *__restrict__ w, int zero_centered,
-                                                                 float *__restrict__ y, int8_t *__restrict__ q,
-                                                                 float *__restrict__ sc, int *bad) {
+// One block per row of d floats (d % 64 == 0, d <= 1024 NV): thread t holds
+// columns 4t .. 4t + 3 of every 1024-column chunk in registers, so the row and
+// the gains are read once. The squares go to LDS, where one wave adds them in row
+// order as pplx_flash/cpu.rs:310-333 does (ordered_sum: the serial loop's bits),
+// and the row scale is 1 / sqrt(ss / d + eps). Then v = (x * scale) * (1 + w)
+// (w when not zero-centred), written to y when y is set, and the A8 codes and
+// scale of each 64-column group (16 consecutive lanes) exactly as
+// act_quantize_kernel computes them from v (int8.rs:178-202), so a product of
+// these codes equals the product of y. A non-finite v sets *bad.
+//
+// Bound by that wave's sum and the launch, not by memory: 8.7 us at 229 rows of
+// 2560 and 10.8 us at 1024, where a serial chain per row in one kernel (12.3 us
+// at either) and this epilogue in a second took 17 us. The sum in a wave of
+// another SIMD for each block of a compute unit was no faster (11.2 us at 1024).
+template <int NV>
+__global__ __launch_bounds__(256) void rms_quantize_kernel(const float *__restrict__ h, int d,
+                                                           const float *__restrict__ w, float eps, int zero_centered,
+                                                           float *__restrict__ y, int8_t *__restrict__ q,
+                                                           float *__restrict__ sc, int *bad) {
+    __shared__ __align__(16) float squares[NV * 1024];
+    __shared__ float scale_sh;
     const size_t row = blockIdx.x, base = row * (size_t)d;
-    const int groups = d / 64;
-    const float scale = sc[row * groups];
-    __syncthreads();  // every thread has the row scale before group 0's scale replaces it
-    // thread t takes columns 4t, 4t + 1, 4t + 2, 4t + 3 of every 1024-column
-    // chunk: a 64-column group is 16 consecutive lanes of one wave. Every
-    // load of the row is in flight before the first group is computed.
-    constexpr int CHUNKS = 4;  // 4096 columns per pass
-    const int lane16 = threadIdx.x % 16;
-    for (int c0 = 0; c0 < d; c0 += CHUNKS * 1024) {
-        float4_t xv[CHUNKS], wv[CHUNKS];
+    const int groups = d / 64, lane16 = threadIdx.x % 16;
+    float4_t xv[NV], wv[NV];
 #pragma unroll
-        for (int u = 0; u < CHUNKS; u++) {
-            const int col = c0 + u * 1024 + 4 * (int)threadIdx.x;
-            xv[u] = col < d ? *(const float4_t *)(h + base + col) : float4_t{0.f, 0.f, 0.f, 0.f};
-            wv[u] = col < d ? *(const float4_t *)(w + col) : float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < NV; u++) {
+        const int col = u * 1024 + 4 * (int)threadIdx.x;
+        xv[u] = col < d ? *(const float4_t *)(h + base + col) : float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+        const int col = u * 1024 + 4 * (int)threadIdx.x;
+        wv[u] = col < d ? *(const float4_t *)(w + col) : float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int u = 0; u < NV; u++)
+        *(float4_t *)(squares + u * 1024 + 4 * threadIdx.x) =
+            float4_t{__fmul_rn(xv[u][0], xv[u][0]), __fmul_rn(xv[u][1], xv[u][1]), __fmul_rn(xv[u][2], xv[u][2]),
+                     __fmul_rn(xv[u][3], xv[u][3])};
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const float ss = ordered_sum(squares, d);
+        if (threadIdx.x == 0) scale_sh = rms_row_scale(ss, d, eps);
+    }
+    __syncthreads();
+    const float scale = scale_sh;
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+        const int col = u * 1024 + 4 * (int)threadIdx.x;
+        if (u * 1024 >= d) break;   // uniform
+        const bool live = col < d;  // the columns of a group are all live or all not
+        float4_t v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float gain = zero_centered ? __fadd_rn(1.0f, wv[u][e]) : wv[u][e];
+            v[e] = __fmul_rn(__fmul_rn(xv[u][e], scale), gain);
         }
+        float maximum = fabsf(v[0]);
 #pragma unroll
-        for (int u = 0; u < CHUNKS; u++) {
-            const int col = c0 + u * 1024 + 4 * (int)threadIdx.x;
-            if (c0 + u * 1024 >= d) break;  // uniform
-            const bool live = col < d;  // the columns of a group are all live or all not
-            float4_t v;
+        for (int e = 1; e < 4; e++) maximum = fmaxf(maximum, fabsf(v[e]));
+        // the group's maximum over its 16 lanes
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float gain = zero_centered ? __fadd_rn(1.0f, wv[u][e]) : wv[u][e];
-                v[e] = __fmul_rn(__fmul_rn(xv[u][e], scale), gain);
-            }
-            float maximum = fabsf(v[0]);
+        for (int off = 8; off > 0; off >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, off, 16));
+        if (!live) continue;
+        if (y) *(float4_t *)(y + base + col) = v;
+        bool finite = true;
 #pragma unroll
-            for (int e = 1; e < 4; e++) maximum = fmaxf(maximum, fabsf(v[e]));
-            // the group's maximum over its 16 lanes
+        for (int e = 0; e < 4; e++) finite = finite && __builtin_isfinite(v[e]);
+        if (!finite && bad) atomicOr(bad, 1);
+        const float s = fmaxf(__fdiv_rn(maximum, 127.0f), FLT_MIN);
+        const float inverse = __frcp_rn(s);
+        uint32_t word = 0;
 #pragma unroll
-            for (int off = 8; off > 0; off >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, off, 16));
-            if (!live) continue;
-            if (y) *(float4_t *)(y + base + col) = v;
-            bool finite = true;
-#pragma unroll
-            for (int e = 0; e < 4; e++) finite = finite && __builtin_isfinite(v[e]);
-            if (!finite && bad) atomicOr(bad, 1);
-            const float s = fmaxf(__fdiv_rn(maximum, 127.0f), FLT_MIN);
-            const float inverse = __frcp_rn(s);
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; e++) word |= (uint32_t)(uint8_t)(int8_t)quantize_code(v[e], inverse, 127.0f) << (8 * e);
-            *(uint32_t *)(q + base + col) = word;
-            if (lane16 == 0) sc[row * groups + col / 64] = s;
-        }
+        for (int e = 0; e < 4; e++) word |= (uint32_t)(uint8_t)(int8_t)quantize_code(v[e], inverse, 127.0f) << (8 * e);
+        *(uint32_t *)(q + base + col) = word;
+        if (lane16 == 0) sc[row * groups + col / 64] = s;
     }
 }
 
@@ -724,9 +641,15 @@ void launch_act_quantize_records(const float *x, int m, int k, uint32_t *records
 void launch_rms_quantize(const float *h, int rows, int d, const float *w, float eps, int zero_centered, float *y,
                          int8_t *q, float *sc, int *bad, hipStream_t s) {
     if (!rows) return;
-    hipLaunchKernelGGL(rms_row_scale_kernel, dim3((unsigned)((rows + kRmsRows - 1) / kRmsRows)), dim3(128), 0, s, h,
-                       rows, d, eps, sc);
-    hipLaunchKernelGGL(rms_apply_quantize_kernel, dim3(rows), dim3(256), 0, s, h, d, w, zero_centered, y, q, sc, bad);
+    static_assert(kRmsQuantizeMaxCols <= 8 * 1024, "the row fits the widest block");
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, s, h, d, w, eps, zero_centered, y, q, sc, bad);
+    };
+    // the smallest that holds the row: registers and LDS follow NV
+    if (d <= 1024) launch(rms_quantize_kernel<1>);
+    else if (d <= 3072) launch(rms_quantize_kernel<3>);
+    else if (d <= 4096) launch(rms_quantize_kernel<4>);
+    else launch(rms_quantize_kernel<8>);
 }
 
 void launch_i8_quantize_rows(const float *x, int rows, int k, int8_t *q, float *scales,
