@@ -2230,25 +2230,31 @@ __global__ __launch_bounds__(WGM *WGN * 64) void grouped_pipe_kernel(
 // WN = 2 the waves are paired along N instead (wave tile 64 rows x 32 columns
 // of each weight): a weight fragment is unpacked once for four row blocks
 // rather than two, and the row maximum takes one exchange through LDS between
-// the pair.
-template <int BM, int WN = 1>
-__global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
+// the pair. BM = 64 with WN = 4 (wave tile 64 rows x 16 columns of each weight)
+// is what the products run: it is bound by the fold's VALU work (three
+// operations per output, group and weight) and, on small grids, by the
+// dependent steps of one wave, so it takes few enough registers for four waves
+// per SIMD (126; reading a step's scales or codes at once takes 130 and the
+// fourth wave) and orders dots before folds (fold_step). Two more load stages
+// changed nothing.
+template <int BM, int WN = 1, int WM = BM / (32 * WN)>
+__global__ __launch_bounds__(WM *WN * 64) void mlp_pipe_kernel(
     const uint8_t *__restrict__ gcodes, const uint8_t *__restrict__ gscales, const uint8_t *__restrict__ ucodes,
     const uint8_t *__restrict__ uscales, const int8_t *__restrict__ q, const float *__restrict__ sx, int m, int n,
     int groups, int kbs, int8_t *__restrict__ qo, float *__restrict__ so, const int *__restrict__ bad) {
-    static_assert(BM == 256 || BM == 128, "8 or 4 waves");
-    static_assert(WN == 1 || WN == 2, "one or two waves across the 64 columns");
-    constexpr int WAVES = BM / 32, MB = 2 * WN, NT = 4 / WN, WR = 32 * WN;
+    static_assert(WN == 1 || WN == 2 || WN == 4, "one, two or four waves across the 64 columns");
+    constexpr int WAVES = WM * WN, WR = BM / WM, MB = WR / 16, NT = 4 / WN;
     constexpr int XSTAGE = BM * 128;   // activation codes, 2 groups per step
     constexpr int CSTAGE = 8 * 1024;   // gate tiles 0-3, up tiles 0-3: one tile16x128 chunk each
     constexpr int SWSTAGE = 2 * 512;   // scale records: [weight][4 tiles x 128 B]
     constexpr int SXSTAGE = BM * 8;
     constexpr int XPW = BM / 8 / WAVES;
+    static_assert(MB * 16 * WM == BM && BM / 32 <= WAVES && XPW % 2 == 0, "whole loads, dealt evenly");
     __shared__ __align__(16) uint8_t xs[2 * XSTAGE];
     __shared__ __align__(16) uint8_t cs[2 * CSTAGE];
     __shared__ __align__(16) uint8_t sws[2 * SWSTAGE];
     __shared__ __align__(16) uint8_t sxs[2 * SXSTAGE];
-    __shared__ float pair_max[WN == 2 ? BM * 2 : 1];
+    __shared__ float part_max[WN > 1 ? BM * WN : 1];
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const int wm = wave / WN, wn = wave % WN;
@@ -2294,7 +2300,7 @@ __global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
             if (wave == 0) dma16(lds, off, live ? rwg : zero_len(rwg));
             else dma16(lds, off, live ? rwu : zero_len(rwu));
         }
-        {
+        if (wave < BM / 32) {  // 32 rows' scales per load
             const int r = wave * 32 + lane / 2;
             dma4(__builtin_amdgcn_readfirstlane(sxs_lds + stage * SXSTAGE + wave * 256),
                  (uint32_t)((r * groups + 2 * st + (lane & 1)) * 4), live ? rs : zero_len(rs));
@@ -2353,6 +2359,74 @@ __global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
         }
     };
 
+    // A wave of one 16-column tile of each weight: a row block's dots are taken
+    // before the fold of the row block before it, so neither waits for the other,
+    // and the second group's activations are read under the first's folds.
+    auto fold_step = [&](const uint8_t *xst, const uint8_t *cst, const uint8_t *swst, const uint8_t *sxst, bool both)
+                         __attribute__((always_inline)) {
+        auto x_frag = [&](int mb, int gp) __attribute__((always_inline)) {
+            const int r = wm * WR + mb * 16 + j, c1 = 4 * gp + qd / 2, c2 = c1 + 2;
+            const uint2_t a0 = *(const uint2_t *)(xst + r * 128 + ((c1 ^ ((r >> 1) & 7)) * 16) + 8 * (qd & 1));
+            const uint2_t a1 = *(const uint2_t *)(xst + r * 128 + ((c2 ^ ((r >> 1) & 7)) * 16) + 8 * (qd & 1));
+            return int4_t{(int)a0[0], (int)a0[1], (int)a1[0], (int)a1[1]};
+        };
+        int4_t xf[MB];
+        float sxv[MB];
+        auto x_scale = [&](int mb, int gp) __attribute__((always_inline)) {
+            return *(const float *)(sxst + (wm * WR + mb * 16 + j) * 8 + gp * 4);
+        };
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            xf[mb] = x_frag(mb, 0);
+            sxv[mb] = x_scale(mb, 0);
+        }
+        int4_t wf[2], d[2][2];  // [weight], [row block parity][weight]
+        float4_t sv[2];
+        auto weights = [&](int gp) __attribute__((always_inline)) {
+#pragma unroll
+            for (int wgt = 0; wgt < 2; wgt++) {
+                const uint2_t wds = *(const uint2_t *)(cst + (wgt * 4 + wn) * 1024 + lane * 16 + gp * 8);
+                const uint2_t lo = nibbles_to_i8x16(wds[0]), hi = nibbles_to_i8x16(wds[1]);
+                wf[wgt] = int4_t{(int)lo[0], (int)lo[1], (int)hi[0], (int)hi[1]};  // 16 * code
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    sv[wgt][v] = *(const float *)(swst + wgt * 512 + wn * 128 + qd * 32 + v * 8 + gp * 4);
+            }
+        };
+        auto dots = [&](int mb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int wgt = 0; wgt < 2; wgt++) d[mb % 2][wgt] = mfma_i8_biased16(wf[wgt], xf[mb]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto fold = [&](int mb) __attribute__((always_inline)) {
+#pragma unroll
+            for (int wgt = 0; wgt < 2; wgt++) {
+                float4_t &out = wgt ? ua[mb][0] : ga[mb][0];
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    out[v] = __builtin_fmaf(dot_value16(d[mb % 2][wgt][v]), __fmul_rn(sv[wgt][v], sxv[mb]), out[v]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        weights(0);
+        dots(0);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            if (mb + 1 < MB) dots(mb + 1);
+            xf[mb] = x_frag(mb, 1);  // of no use past the last group, but in the stage
+            fold(mb);
+            sxv[mb] = x_scale(mb, 1);
+        }
+        if (!both) return;
+        weights(1);
+        dots(0);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            if (mb + 1 < MB) dots(mb + 1);
+            fold(mb);
+        }
+    };
+
     if (!nan_out) {
         // unrolled by the two stages: every LDS address is a fixed per-lane offset plus an immediate
         auto run_step = [&](auto stage, int st) {
@@ -2362,8 +2436,12 @@ __global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
             load_stage(C ^ 1, st + 1, st + 1 < steps);
             const uint8_t *xst = xs + C * XSTAGE, *cst = cs + C * CSTAGE;
             const uint8_t *swst = sws + C * SWSTAGE, *sxst = sxs + C * SXSTAGE;
-            fold_group(xst, cst, swst, sxst, 0);
-            if (2 * st + 1 < groups) fold_group(xst, cst, swst, sxst, 1);
+            if constexpr (NT == 1) {
+                fold_step(xst, cst, swst, sxst, 2 * st + 1 < groups);
+            } else {
+                fold_group(xst, cst, swst, sxst, 0);
+                if (2 * st + 1 < groups) fold_group(xst, cst, swst, sxst, 1);
+            }
         };
         load_stage(0, 0, true);
         for (int st = 0; st < steps; st += 2) {
@@ -2393,13 +2471,16 @@ __global__ __launch_bounds__(BM / 32 * 64) void mlp_pipe_kernel(
         local = fmaxf(local, __shfl_xor(local, 32));
         rmax[mb] = local;
     }
-    if (WN == 2) {  // the other half of each row's columns is in the paired wave
+    if (WN > 1) {  // the rest of each row's columns is in the other waves of the row
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
-            if (qd == 0) pair_max[(wm * WR + mb * 16 + j) * 2 + wn] = rmax[mb];
+            if (qd == 0) part_max[(wm * WR + mb * 16 + j) * WN + wn] = rmax[mb];
         __syncthreads();
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) rmax[mb] = fmaxf(rmax[mb], pair_max[(wm * WR + mb * 16 + j) * 2 + (wn ^ 1)]);
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int o = 1; o < WN; o++)
+                rmax[mb] = fmaxf(rmax[mb], part_max[(wm * WR + mb * 16 + j) * WN + (wn ^ o)]);
     }
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
@@ -2438,8 +2519,9 @@ const char *const kI8Names[] = {"256x256p2w8", "256x256p4k64w8", "256x128p3w8", 
 const char *const kGroupedNames[] = {"pipe-auto",    "pipe256x128w8", "wave16x16",   "pipe128x128w4",
                                      "pipe64x128w2", "pipe128x128m8", "pipe128x128n8", "pipe32x128w8",
                                      "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16",
-                                     "pipe32x64w4",  "pipe64x64w8"};
-const char *const kMlpNames[] = {"pipe-auto", "pipe256x64w8", "pipe128x64w4", "wave16x64", "pipe256x64n2", "pipe128x64n2"};
+                                     "pipe32x64w4",  "pipe64x64w8",  "pipe32x64w4g4", "pipe16x64w4g4"};
+const char *const kMlpNames[] = {"pipe-auto", "pipe256x64w8", "pipe128x64w4", "wave16x64", "pipe256x64n2", "pipe128x64n2",
+                                  "pipe64x64n4"};
 const char *const kDeltaNames[] = {"chunked64", "chunked64-c32", "recurrent", "recurrent-rolled", "auto"};
 const char *const kNormNames[] = {"fused", "separate"};
 
@@ -2726,8 +2808,8 @@ int variant_count(const char *family) {
     if (f == "gemv") return 6;
     if (f == "gemm_w4a16") return 14;
     if (f == "i8_gemm") return 13;
-    if (f == "grouped") return 14;
-    if (f == "mlp") return 6;
+    if (f == "grouped") return 16;
+    if (f == "mlp") return 7;
     if (f == "delta_scan") return 5;
     if (f == "norm") return 2;
     return 0;
@@ -2820,13 +2902,14 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 // one wave per 16x16 tile; 9 and 10 are 7 and 8 with four groups per k-step
 // instead of two; 11 the few-row kernel over the codes (16 rows per block
 // row, a block per 16 columns); 12 and 13 are 32x64 tiles on 4 waves (each
-// 32 rows x 16 columns, the per-wave work of 7) and 64x64 on 8 waves. Every
+// 32 rows x 16 columns, the per-wave work of 7) and 64x64 on 8 waves; 14 and
+// 15 are 32x64 and 16x64 tiles on 4 waves with four groups per k-step. Every
 // variant folds in group order: all are bitwise equal. "Auto" (0) picks:
-//  - the few-row kernel where its grid gives a compute unit at most two
-//    blocks (us, A8 codes in: K=9216, N=2560, 17-48 rows: 19.9-21.7 against
-//    27.6 pipelined; N=1024, 17-128 rows: 4.8-8.3 against 10.0; N=4096,
-//    17-32 rows: 8.1 against 9.8; one block row more and it is slower), not
-//    for affine weights, which it does not take;
+//  - the few-row kernel where its grid gives a compute unit at most one block
+//    (us, few-row / 16x64w4g4: N=1024, K=9216, 64 rows 20.0 / 25.9; K=4096
+//    12.0 / 15.3; K=2560 10.6 / 12.3; with two blocks it loses: N=1024, K=2560,
+//    128 rows 15.3 / 12.6; N=2560, K=9216, 48 rows 33.0 / 26.3), not for affine
+//    weights, which it does not take;
 //  - otherwise, as the fold is VALU work, the tiles whose grid keeps every
 //    SIMD busy and every compute unit equally loaded: where a grid's blocks
 //    do not divide evenly over the units, those holding one block more end
@@ -2834,9 +2917,16 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 //    the rest; 1280 32x64 blocks put five on each). So 128x128 side by side
 //    when their grid gives every unit four blocks, else 64x128 on 8 waves
 //    when its grid is two or more whole blocks per unit, else 32x64 on 4
-//    waves, and 32x128 with four groups per step when the 32x128 grid gives
-//    a unit fewer than two blocks (half the barriers and twice the work
-//    between a load and its use; on fuller grids it is 2-5% slower).
+//    waves; a grid too small for that is bound by the chain of steps of one
+//    block, so it takes four groups per step (half the barriers and twice the
+//    work between a load and its use; on fuller grids that is 2-5% slower) and
+//    the tile with the shortest step: 16x64 up to two and a half blocks per
+//    unit, else 32x64.
+// Measured there (us, 32x128w8g4 / 32x64w4g4 / 16x64w4g4 at 40, 128, 192 rows):
+// N=2560, K=9216 33.4 / 30.2 / 26.2, 35.5 / 32.8 / 28.8, 37.0 / 34.5 / 30.6;
+// N=2560, K=4096 19.1 / 17.2 / 15.4, 21.4 / 18.4 / 16.9, 21.4 / 19.9 / 18.0;
+// N=4160, K=2560 15.6 / 14.3 / 13.3, 16.5 / 15.9 / 15.3, 17.1 / 16.9 / 18.1;
+// N=8192, K=2560 15.8 / 14.6 / 13.7, 17.2 / 17.0 / 18.6, 22.5 / 20.7 / 24.1.
 // Measured (us at 1024 rows unless stated; 32x128w8 / 32x128w8g4 / 32x64w4 /
 // 64x128w8 / 128x128 side by side): N=1024, K=2560 18.0 / 16.3 / 17.1 / 22.0
 // / 47.5; N=2560, K=9216 79.0 / 82.7 / 74.6 / 83.9 / 149; N=2560, K=4096
@@ -2847,12 +2937,12 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 int grouped_pick(const Weight &w, int m, int variant) {
     if (variant != 0) return variant;
     const unsigned cus = (unsigned)device_cus(), tn = cdiv(w.rows, 128);
-    if (!w.offsets && cdiv(m, 16) * (unsigned)w.tiles() <= 2 * cus) return 11;
+    if (!w.offsets && cdiv(m, 16) * (unsigned)w.tiles() <= cus) return 11;
     if (cdiv(m, 128) * tn >= 4 * cus) return 5;
     const unsigned b64 = cdiv(m, 64) * tn;
     if (b64 >= 2 * cus && b64 % cus == 0) return 8;
     if (cdiv(m, 32) * tn >= 2 * cus) return 12;
-    return 9;
+    return 2 * cdiv(m, 16) * cdiv(w.rows, 64) < 5 * cus ? 15 : 14;
 }
 
 // Activation rows per block of a pipelined pick (0: not a pipelined kernel).
@@ -2861,7 +2951,8 @@ int grouped_pipe_rows(int pick) {
         case 1: return 256;
         case 3: case 5: case 6: return 128;
         case 4: case 8: case 10: case 13: return 64;
-        case 7: case 9: case 12: return 32;
+        case 7: case 9: case 12: case 14: return 32;
+        case 15: return 16;
         default: return 0;
     }
 }
@@ -2889,6 +2980,8 @@ bool launch_grouped(const Weight &w, const int8_t *q, const float *sx, int m, fl
         case 10: if (grouped_pipe_launch<64, 2, 4, 4>(w, q, sx, m, y, bad, s, res, sxq)) return true; break;
         case 12: if (grouped_pipe_launch<32, 1, 4, 2, 64>(w, q, sx, m, y, bad, s, res, sxq)) return true; break;
         case 13: if (grouped_pipe_launch<64, 2, 4, 2, 64>(w, q, sx, m, y, bad, s, res, sxq)) return true; break;
+        case 14: if (grouped_pipe_launch<32, 1, 4, 4, 64>(w, q, sx, m, y, bad, s, res, sxq)) return true; break;
+        case 15: if (grouped_pipe_launch<16, 1, 4, 4, 64>(w, q, sx, m, y, bad, s, res, sxq)) return true; break;
         case 11:
             if (w.offsets) break;  // the few-row kernel over codes takes no offsets
             if (w.bits == 4) gv_launch_m<4, 1, false>(w, q, sx, m, 8, y, bad, nullptr, s, res);
@@ -2911,52 +3004,36 @@ bool launch_grouped(const Weight &w, const int8_t *q, const float *sx, int m, fl
 }
 
 // Variants: 1 pipelined 256x64 blocks (8 waves), 2 128x64 blocks (4 waves),
-// 4 and 5 the same blocks with the waves paired along N (wave tile 64 x 32), 3
-// one wave per 16x64 block. 0 picks the paired 256-row blocks when their grid
-// covers half the compute units but not all of them and has fewer blocks than
-// the 128-row grid (not at m <= 128, where the 256-row blocks are half empty:
-// 54 against 40 us at M = 128, K = 2560, N = 9216), else the paired 128-row
-// blocks when theirs covers half, else the one-wave blocks (measured at K=2560,
-// N=9216: the paired layouts are 7-16% faster than the stacked ones at every M
-// from 229 to 4096, and 128-row blocks beat 256-row blocks from M=1024 up).
+// 4 and 5 the same blocks with the waves paired along N (wave tile 64 x 32), 6
+// 64x64 blocks with four waves along N (wave tile 64 x 16), 3 one wave per
+// 16x64 block. 0 picks the 64-row blocks: the most waves a unit holds, the
+// finest grid of the pipelined forms and the shortest step. Measured (us with
+// the quantizer, 128-row paired / 64-row): K=2560, N=9216, 64 rows 39.9 / 27.4,
+// 229 rows 53.3 (256-row paired 56.7) / 43.2, 1024 rows 127 / 110, 4096 rows
+// 392 / 385; N=1024, 229 rows 39.8 / 28.1; K=4096, N=14336, 229 rows 79.5 /
+// 76.2, 4096 rows 916 / 901. Up to three rows the one-wave blocks, which read no
+// empty rows (1 row, one-wave / 64-row: N=1024 23.9 / 26.6, K=4096, N=14336 36.4
+// / 38.9; at 4 rows 26.9 / 26.4 and 43.8 / 38.6).
 // All variants are word-exact with the unfused composition.
 void launch_mlp_requant(const Weight &gate, const Weight &up, const int8_t *q, const float *sx,
                         int m, int8_t *qo, float *so, const int *bad, int variant, hipStream_t s) {
     if (m == 0) return;
-    const unsigned cus = (unsigned)device_cus(), tn = (unsigned)(gate.rows / 64);
+    const unsigned tn = (unsigned)(gate.rows / 64);
     const bool fits = (size_t)256 * gate.groups * 64 < ((size_t)1 << 31) &&
                       (size_t)4 * gate.kblocks() * 1024 < ((size_t)1 << 31) && ((uintptr_t)qo & 3) == 0 &&
                       gate.rows % 4 == 0;
-    int pick = variant;
-    if (variant == 0) {
-        // 256-row blocks only where they shorten the grid (at m <= 128 both
-        // grids have the same blocks, half of each 256-row block empty)
-        const unsigned b256 = cdiv(m, 256) * tn, b128 = cdiv(m, 128) * tn;
-        if (2 * b256 >= cus && b256 < cus && b256 < b128) pick = 4;
-        else if (2 * b128 >= cus) pick = 5;
-        else pick = 3;
-    }
-    if (fits && pick == 1) {
-        hipLaunchKernelGGL(mlp_pipe_kernel<256>, dim3(cdiv(m, 256) * tn), dim3(512), 0, s, gate.codes, gate.scales,
-                           up.codes, up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo, so, bad);
-        return;
-    }
-    if (fits && pick == 2) {
-        hipLaunchKernelGGL(mlp_pipe_kernel<128>, dim3(cdiv(m, 128) * tn), dim3(256), 0, s, gate.codes, gate.scales,
-                           up.codes, up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo, so, bad);
-        return;
-    }
-    if (fits && pick == 4) {
-        hipLaunchKernelGGL((mlp_pipe_kernel<256, 2>), dim3(cdiv(m, 256) * tn), dim3(512), 0, s, gate.codes,
-                           gate.scales, up.codes, up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo,
-                           so, bad);
-        return;
-    }
-    if (fits && pick == 5) {
-        hipLaunchKernelGGL((mlp_pipe_kernel<128, 2>), dim3(cdiv(m, 128) * tn), dim3(256), 0, s, gate.codes,
-                           gate.scales, up.codes, up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo,
-                           so, bad);
-        return;
+    const int pick = variant != 0 ? variant : m < 4 ? 3 : 6;
+    const auto launch = [&](auto kernel, int bm, int waves) {
+        hipLaunchKernelGGL(kernel, dim3(cdiv(m, bm) * tn), dim3(waves * 64), 0, s, gate.codes, gate.scales, up.codes,
+                           up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo, so, bad);
+    };
+    if (fits) switch (pick) {
+        case 1: return launch(mlp_pipe_kernel<256>, 256, 8);
+        case 2: return launch(mlp_pipe_kernel<128>, 128, 4);
+        case 4: return launch(mlp_pipe_kernel<256, 2>, 256, 8);
+        case 5: return launch(mlp_pipe_kernel<128, 2>, 128, 4);
+        case 6: return launch(mlp_pipe_kernel<64, 4, 1>, 64, 4);
+        default: break;
     }
     dim3 grid(gate.rows / 64, cdiv(m, 16));
     hipLaunchKernelGGL(mlp_requant_kernel, grid, dim3(256), 0, s, gate.codes, gate.scales, up.codes,

@@ -124,3 +124,53 @@ def test_i8_row_quantizer_of_every_width(ctx, oracle, k):
     ctx.i8_quantize_rows(dev(x), rows, k, q, s)
     assert np.isinf(host(ctx, s)[2]) and np.array_equal(host(ctx, q)[[0, 1, 3, 4]], wq[[0, 1, 3, 4]])
     assert not host(ctx, q)[2].any()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,k,n", [(17, 64, 16), (31, 320, 63), (33, 576, 65), (48, 192, 200), (129, 1088, 128)])
+def test_grouped_four_group_tiles_give_the_one_wave_kernels_bits(ctx, bits, m, k, n):
+    """The 16x64 and 32x64 tiles with four groups per step: one to seventeen
+    groups (a last step of one, two or three), ragged rows and columns, no
+    store past the output."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(m + n + k + bits)
+    w = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.05).astype(np.float32)), rocm.F32, n, k, bits, 64)
+    x = dev(rng.standard_normal((m, k)).astype(np.float32))
+    out = {}
+    try:
+        for name in ("wave16x16", "pipe32x64w4g4", "pipe16x64w4g4"):
+            ctx.select_variant("grouped", name)
+            y = torch.full((m * n + 64,), -7.0, dtype=torch.float32, device="cuda")
+            torch.cuda.synchronize()
+            ctx.linear(w, x, rocm.F32, m, y, rocm.W4A8)
+            out[name] = host(ctx, y)
+            assert (out[name][m * n:] == -7.0).all(), name
+    finally:
+        ctx.select_variant("grouped", "pipe-auto")
+    for name in out:
+        assert bits_equal(out[name], out["wave16x16"]), name
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 64), (3, 128, 64), (4, 192, 128), (63, 320, 64), (65, 1088, 192), (129, 576, 64)])
+def test_mlp_64_row_blocks_give_the_one_wave_kernels_bits(ctx, m, k, n):
+    """The fused MLP's 64x64 blocks: odd group counts, one group, ragged rows,
+    and the rows where the choice of kernel turns."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(m + n + k)
+    gate, up = (ctx.quantize(dev((rng.standard_normal((n, k)) * 0.05).astype(np.float32)), rocm.F32, n, k, 4, 64)
+                for _ in range(2))
+    x = dev((rng.standard_normal((m, k)) * 1.3).astype(np.float32))
+    out = {}
+    try:
+        for name in ("wave16x64", "pipe64x64n4", "pipe-auto"):
+            ctx.select_variant("mlp", name)
+            q = torch.full((m * n + 64,), 99, dtype=torch.int8, device="cuda")
+            s = torch.full((m * n // 64 + 16,), -7.0, dtype=torch.float32, device="cuda")
+            torch.cuda.synchronize()
+            ctx.mlp_requant(gate, up, x, m, q, s)
+            out[name] = host(ctx, q), host(ctx, s)
+            assert (out[name][0][m * n:] == 99).all() and (out[name][1][m * n // 64:] == -7.0).all(), name
+    finally:
+        ctx.select_variant("mlp", "pipe-auto")
+    for name in out:
+        assert np.array_equal(out[name][0], out["wave16x64"][0]) and bits_equal(out[name][1], out["wave16x64"][1]), name
