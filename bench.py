@@ -537,7 +537,7 @@ def pplx_line(torch, ctx, rocm, stream, n: int = 1024, layers: int = 32) -> dict
 TUNE_SHAPES = {"grouped": (256, 8192, 2560), "mlp": (128, 9216, 2560), "gemv": (1, 8192, 2560),
                "gemm_w4a16": (256, 8192, 2560), "i8_gemm": (256, 8192, 2560)}
 TUNE_REFERENCE = {"grouped": "pipe-auto", "mlp": "pipe-auto", "gemv": "auto", "gemm_w4a16": "pipe-auto",
-                  "i8_gemm": "256x256p2w8"}
+                  "i8_gemm": "auto"}
 
 
 def tune_line(torch, ctx, rocm, stream, budget_ms: int, cache_in: str | None, cache_out: str | None,

@@ -2511,11 +2511,10 @@ const char *const kGemmNames[] = {"pipe-auto",   "256x256p2w8", "128x128p2w4", "
                                    "256x128w2x2", "128x128w2x2", "128x64w2x2", "256x256p2w8-persist",
                                    "256x192p2w8-persist", "256x128p2w8", "small32x32",
                                    "small32x64", "small64x64", "small64x128"};
-const char *const kI8Names[] = {"256x256p2w8", "256x256p4k64w8", "256x128p3w8", "256x128p3",
+const char *const kI8Names[] = {"auto", "256x256p4k64w8", "256x128p3w8", "256x128p3",
                                  "128x128w2x2", "256x128w2x2", "64x64w2x2", "256x256p2w8-stream",
                                  "256x256p2w8-stream-mid", "256x128k64p2-stream2",
-                                 "rows",
-                                 "64x64p4", "128x128p3w8"};
+                                 "256x256p2w8", "rows", "64x64p4", "128x128p3w8"};
 const char *const kGroupedNames[] = {"pipe-auto",    "pipe256x128w8", "wave16x16",   "pipe128x128w4",
                                      "pipe64x128w2", "pipe128x128m8", "pipe128x128n8", "pipe32x128w8",
                                      "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16",
@@ -2807,7 +2806,7 @@ int variant_count(const char *family) {
     std::string f(family);
     if (f == "gemv") return 6;
     if (f == "gemm_w4a16") return 14;
-    if (f == "i8_gemm") return 13;
+    if (f == "i8_gemm") return 14;
     if (f == "grouped") return 16;
     if (f == "mlp") return 7;
     if (f == "delta_scan") return 5;
@@ -3110,11 +3109,11 @@ bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, 
     return true;
 }
 
-// Variant 0 picks among the pipelined buffer-to-LDS kernels by the grid; 1-3
-// are fixed ones and 7-9 their persistent stream form (int8 B, k % 16 == 0);
-// 10 streams the weight for a few rows (i8_rows_kernel), 11 and 12 are small
-// tiles; 4-6 stage through registers and take any k and the per-row Q4 B
-// operand. Variant 0 takes the first that fits (us, graph-timed; rows /
+// Variant 0 ("auto") picks among the pipelined buffer-to-LDS kernels by the
+// grid; 1-3 and 10 are fixed ones and 7-9 their persistent stream form (int8 B,
+// k % 16 == 0); 11 streams the weight for a few rows (i8_rows_kernel), 12 and
+// 13 are small tiles; 4-6 stage through registers and take any k and the
+// per-row Q4 B operand. Variant 0 takes the first that fits (us, graph-timed; rows /
 // 64x64p4 / 128x128p3w8 / 256x128p3w8 / 256x256p2w8):
 //  - the rows kernel up to 32 rows where its grid is one block per unit or
 //    less (K=N=4096: 1 row 6.3 / 12.2 / 17.2 / 26.2 / 40.1, 32 rows 9.3 / 12.5,
@@ -3159,9 +3158,10 @@ void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, 
             case 7: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 8: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, true>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 9: if (i8_stream_launch<256, 128, 64, 2, 2, 2, 2, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 10: if (launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 11: if (i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 12: if (i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 10: if (i8_pipe_launch<256, 256, 128, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 11: if (launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 12: if (i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 13: if (i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             default: break;
         }
     }

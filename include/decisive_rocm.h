@@ -584,10 +584,14 @@ int32_t dz_tune(dz_ctx *ctx, uint32_t budget_ms, const char *cache_in, char *cac
  *   "gemm_w4a16"  pipe-auto, 256x256p2w8, 128x128p2w4, 128x256p2w8, 256x128w2x2,
  *                 128x128w2x2, 128x64w2x2, 256x256p2w8-persist, 256x192p2w8-persist,
  *                 256x128p2w8
- *   "i8_gemm"     256x256p2w8, 256x256p4k64w8, 256x128p3w8, 256x128p3, 128x128w2x2,
+ *   "i8_gemm"     auto, 256x256p4k64w8, 256x128p3w8, 256x128p3, 128x128w2x2,
  *                 256x128w2x2, 64x64w2x2, 256x256p2w8-stream, 256x256p2w8-stream-mid,
  *                 256x128k64p2-stream2 (the "-stream" forms are persistent: one
- *                 or two blocks per compute unit, each walking several tiles)
+ *                 or two blocks per compute unit, each walking several tiles),
+ *                 256x256p2w8, rows (the weight streamed over up to 32 rows at a
+ *                 time), 64x64p4, 128x128p3w8; "auto" takes rows, 64x64p4,
+ *                 128x128p3w8, 256x128p3w8 or 256x256p2w8 by the grid, and a
+ *                 variant that cannot take a shape runs 128x128w2x2
  *   "grouped"     pipe-auto, pipe256x128w8, wave16x16, pipe128x128w4, pipe64x128w2,
  *                 pipe128x128m8, pipe128x128n8, pipe32x128w8, pipe64x128w8,
  *                 pipe32x128w8g4, pipe64x128w8g4 (g4: four 64-groups per

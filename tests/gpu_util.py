@@ -38,3 +38,15 @@ def cosine(a, b):
     a = np.asarray(a, np.float64).reshape(-1)
     b = np.asarray(b, np.float64).reshape(-1)
     return float(a @ b / (np.linalg.norm(a) * np.linalg.norm(b) + 1e-300))
+
+
+def launched(ctx, fn):
+    """The names of the kernels that fn() launches on the context's stream."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    ctx.sync()
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as prof:
+        fn()
+        ctx.sync()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events()]

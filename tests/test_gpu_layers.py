@@ -403,5 +403,5 @@ def test_tuned_grouped_and_mlp_variants_agree_on_real_inputs(ctx, oracle):
 
 
 def rocm_reference(fam):
-    return {"gemv": "auto", "gemm_w4a16": "pipe-auto", "i8_gemm": "256x256p2w8", "grouped": "pipe-auto",
+    return {"gemv": "auto", "gemm_w4a16": "pipe-auto", "i8_gemm": "auto", "grouped": "pipe-auto",
             "mlp": "pipe-auto", "norm": "fused", "delta_scan": "chunked64"}[fam]

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from decisive_amd import rocm
-from tests.gpu_util import bits_equal, cosine, dev, empty, host
+from tests.gpu_util import bits_equal, cosine, dev, empty, host, launched
 
 pytestmark = pytest.mark.gpu
 GOLDEN = json.loads((Path(__file__).parent / "golden" / "reference_vectors.json").read_text())
@@ -610,8 +610,9 @@ def test_config5_prefill_rows_vs_fp32(ctx, oracle):
 
 # ---- per-row int8 ----------------------------------------------------------------------
 
-I8_VARIANTS = ("256x256p2w8", "256x256p4k64w8", "256x128p3w8", "256x128p3", "128x128w2x2", "256x128w2x2",
-               "64x64w2x2", "256x256p2w8-stream", "256x256p2w8-stream-mid", "256x128k64p2-stream2")
+I8_VARIANTS = ("auto", "256x256p4k64w8", "256x128p3w8", "256x128p3", "128x128w2x2", "256x128w2x2",
+               "64x64w2x2", "256x256p2w8-stream", "256x256p2w8-stream-mid", "256x128k64p2-stream2", "256x256p2w8",
+               "rows", "64x64p4", "128x128p3w8")
 
 
 @pytest.mark.parametrize("m,n,k", GOLDEN["q4_raw_check_shapes"]["mnk"] + [[77, 45, 100], [1, 1, 4], [130, 260, 4100],
@@ -636,6 +637,25 @@ def test_i8_gemm_exact(ctx, oracle, m, n, k):
         assert np.array_equal(host(ctx, r), raw), name
         assert bits_equal(host(ctx, y), yf), name
     ctx.select_variant("i8_gemm", I8_VARIANTS[0])
+
+
+def test_i8_variant_names_run_their_kernels(ctx):
+    """The default is the rule that picks by the grid; a tile named runs that
+    tile, at sizes where the rule takes another."""
+    torch = pytest.importorskip("torch")
+    m, n, k = 300, 520, 4112
+    a, b = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda") for s in ((m, k), (n, k)))
+    y = empty((m, n), torch.int32)
+    assert ctx.info()["variants"]["i8_gemm"] == "auto"
+    tiles = {"auto": "64, 64, 128, 4", "256x256p2w8": "256, 256, 128, 2", "256x128p3w8": "256, 128, 128, 3",
+             "64x64p4": "64, 64, 128, 4", "128x128p3w8": "128, 128, 128, 3"}
+    try:
+        for name, args in tiles.items():
+            ctx.select_variant("i8_gemm", name)
+            got = launched(ctx, lambda: ctx.i8_gemm(a, None, m, b, None, n, k, y, raw=True))
+            assert any(f"i8_gemm_pipe_kernel<{args}," in g for g in got), (name, got)
+    finally:
+        ctx.select_variant("i8_gemm", "auto")
 
 
 @pytest.mark.parametrize("m,n,k", [[1, 1, 4], [77, 45, 100], [130, 260, 4100], [256, 512, 4096], [513, 257, 80]])

@@ -92,7 +92,7 @@ def test_i8_products_of_every_size_are_exact(ctx, m, n, k):
     want = ((dots.astype(np.float32) * sa[:, None]).astype(np.float32) * sb).astype(np.float32)
     da, db, dsa, dsb = dev(a), dev(b), dev(sa), dev(sb)
     try:
-        for name in ("256x256p2w8", "rows", "64x64p4", "128x128p3w8"):
+        for name in ("auto", "256x256p2w8", "rows", "64x64p4", "128x128p3w8"):
             ctx.select_variant("i8_gemm", name)
             r = torch.full((m * n + 64,), -7, dtype=torch.int32, device="cuda")
             y = torch.full((m * n + 64,), -7.0, dtype=torch.float32, device="cuda")
@@ -104,7 +104,7 @@ def test_i8_products_of_every_size_are_exact(ctx, m, n, k):
             assert bits_equal(f[:m * n].reshape(m, n), want), name
             assert (raw[m * n:] == -7).all() and (f[m * n:] == -7.0).all(), name
     finally:
-        ctx.select_variant("i8_gemm", "256x256p2w8")
+        ctx.select_variant("i8_gemm", "auto")
 
 
 @pytest.mark.parametrize("k", [4, 6, 1024, 1028, 2052, 4096, 8196, 16388, 32768])
