@@ -3095,6 +3095,14 @@ bool i8_pipe_launch(const int8_t *a, const float *sa, int m, const int8_t *b, co
     return true;
 }
 
+// A tile in its ragged form where k is not whole 16-byte chunks.
+template <int BM, int BN, int NS, int WGM, int WGN>
+bool i8_any_k_launch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k, void *y,
+                     int raw, hipStream_t s) {
+    return k % 16 != 0 ? i8_pipe_launch<BM, BN, 128, NS, WGM, WGN, true>(a, sa, m, b, sb, n, k, y, raw, s)
+                       : i8_pipe_launch<BM, BN, 128, NS, WGM, WGN>(a, sa, m, b, sb, n, k, y, raw, s);
+}
+
 // BPC blocks per compute unit (what the kernel's LDS and registers allow).
 template <int BM, int BN, int BK, int NS, int WGM, int WGN, int BPC, bool MID>
 bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n, int k,
@@ -3110,10 +3118,11 @@ bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, 
 }
 
 // Variant 0 ("auto") picks among the pipelined buffer-to-LDS kernels by the
-// grid; 1-3 and 10 are fixed ones and 7-9 their persistent stream form (int8 B,
-// k % 16 == 0); 11 streams the weight for a few rows (i8_rows_kernel), 12 and
-// 13 are small tiles; 4-6 stage through registers and take any k and the
-// per-row Q4 B operand. Variant 0 takes the first that fits (us, graph-timed; rows /
+// grid; 1-3 are fixed ones and 7-9 their persistent stream form (int8 B,
+// k % 16 == 0); 10 is the 256x256 tile, 11 streams the weight for a few rows
+// (i8_rows_kernel), 12 and 13 are small tiles (10 to 13 take k % 4 == 0); 4-6
+// stage through registers and take any k and the per-row Q4 B operand.
+// Variant 0 takes the first that fits (us, graph-timed; rows /
 // 64x64p4 / 128x128p3w8 / 256x128p3w8 / 256x256p2w8):
 //  - the rows kernel up to 32 rows where its grid is one block per unit or
 //    less (K=N=4096: 1 row 6.3 / 12.2 / 17.2 / 26.2 / 40.1, 32 rows 9.3 / 12.5,
@@ -3123,8 +3132,8 @@ bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, 
 //  - 128x128, then 256x128, where their grid fits one wave of units (1024
 //    rows 37.5 / 27.8 / 33.5 / 45.6, 2048 rows 68.7 / 52.1 / 45.6 / 52.2);
 //  - 256x256 (4096 rows 125.9 / 94.2 / 81.8 / 70.9).
-// Where k % 16 != 0 the ragged forms of 64x64, 128x128 and 256x256 take k % 4
-// == 0, and any other k is staged: on 64x64 tiles up to three 128x128 blocks
+// Where k % 16 != 0 the ragged forms of 64x64, 128x128 and 256x256 (also in
+// 256x128's place) take k % 4 == 0, and any other k is staged: on 64x64 tiles up to three 128x128 blocks
 // for every two units (K=1000, N=1063, 300 rows 16.1 against 32.6), 128x128
 // beyond. Every variant computes exact int32 dots, so all are bitwise equal;
 // when a pipelined variant cannot take a shape, the register-staged 128x128 runs.
@@ -3138,18 +3147,10 @@ void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, 
         switch (variant) {
             case 0:
                 if (m <= 32 && cdiv(n, 16) <= cus && launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return;
-                if (k % 16 != 0) {
-                    if (few64 ? i8_pipe_launch<64, 64, 128, 4, 2, 2, true>(a, sa, m, b, sb, n, k, y, raw, s)
-                        : grid(128, 128) <= cus
-                            ? i8_pipe_launch<128, 128, 128, 3, 2, 4, true>(a, sa, m, b, sb, n, k, y, raw, s)
-                            : i8_pipe_launch<256, 256, 128, 2, 2, 4, true>(a, sa, m, b, sb, n, k, y, raw, s))
-                        return;
-                    break;
-                }
-                if (few64 ? i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)
-                    : grid(128, 128) <= cus ? i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
-                    : grid(256, 128) <= cus ? i8_pipe_launch<256, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
-                                            : i8_pipe_launch<256, 256, 128, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s))
+                if (few64                                    ? i8_any_k_launch<64, 64, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)
+                    : grid(128, 128) <= cus                  ? i8_any_k_launch<128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
+                    : k % 16 == 0 && grid(256, 128) <= cus ? i8_pipe_launch<256, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)
+                                                             : i8_any_k_launch<256, 256, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s))
                     return;
                 break;
             case 1: if (i8_pipe_launch<256, 256, 64, 4, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
@@ -3158,10 +3159,10 @@ void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, 
             case 7: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 8: if (i8_stream_launch<256, 256, 128, 2, 2, 4, 1, true>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 9: if (i8_stream_launch<256, 128, 64, 2, 2, 2, 2, false>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 10: if (i8_pipe_launch<256, 256, 128, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 10: if (i8_any_k_launch<256, 256, 2, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             case 11: if (launch_i8_rows(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 12: if (i8_pipe_launch<64, 64, 128, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
-            case 13: if (i8_pipe_launch<128, 128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 12: if (i8_any_k_launch<64, 64, 4, 2, 2>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
+            case 13: if (i8_any_k_launch<128, 128, 3, 2, 4>(a, sa, m, b, sb, n, k, y, raw, s)) return; break;
             default: break;
         }
     }

@@ -641,19 +641,22 @@ def test_i8_gemm_exact(ctx, oracle, m, n, k):
 
 def test_i8_variant_names_run_their_kernels(ctx):
     """The default is the rule that picks by the grid; a tile named runs that
-    tile, at sizes where the rule takes another."""
+    tile, at sizes where the rule takes another, and in its ragged form where k
+    is not whole 16-byte chunks."""
     torch = pytest.importorskip("torch")
-    m, n, k = 300, 520, 4112
-    a, b = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda") for s in ((m, k), (n, k)))
-    y = empty((m, n), torch.int32)
     assert ctx.info()["variants"]["i8_gemm"] == "auto"
-    tiles = {"auto": "64, 64, 128, 4", "256x256p2w8": "256, 256, 128, 2", "256x128p3w8": "256, 128, 128, 3",
-             "64x64p4": "64, 64, 128, 4", "128x128p3w8": "128, 128, 128, 3"}
+    tiles = {"256x256p2w8": "256, 256, 128, 2", "64x64p4": "64, 64, 128, 4", "128x128p3w8": "128, 128, 128, 3"}
+    runs = [(300, 520, k, name, args, k == 1004) for k in (4112, 1004) for name, args in tiles.items()]
+    runs += [(300, 520, 4112, "256x128p3w8", "256, 128, 128, 3", False), (300, 520, 4112, "auto", tiles["64x64p4"], False),
+             (300, 520, 1004, "auto", tiles["64x64p4"], True), (1000, 2000, 1004, "auto", tiles["128x128p3w8"], True),
+             (2100, 4100, 132, "auto", tiles["256x256p2w8"], True)]
     try:
-        for name, args in tiles.items():
+        for m, n, k, name, args, ragged in runs:
+            a, b = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda") for s in ((m, k), (n, k)))
+            y = empty((m, n), torch.int32)
             ctx.select_variant("i8_gemm", name)
             got = launched(ctx, lambda: ctx.i8_gemm(a, None, m, b, None, n, k, y, raw=True))
-            assert any(f"i8_gemm_pipe_kernel<{args}," in g for g in got), (name, got)
+            assert any(f"i8_gemm_pipe_kernel<{args}," in g and f"{str(ragged).lower()}>" in g for g in got), (m, n, k, name, got)
     finally:
         ctx.select_variant("i8_gemm", "auto")
 

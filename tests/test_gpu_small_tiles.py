@@ -77,7 +77,9 @@ def test_w4a16_rows_do_not_see_each_other(ctx, k):
 @pytest.mark.parametrize("m,n,k", [
     (1, 1, 4), (16, 16, 64), (17, 33, 68), (32, 47, 508), (33, 64, 512),        # the few-row kernel's edges and chunk tails
     (64, 65, 20), (65, 129, 132), (300, 4096, 260), (129, 1000, 516),           # small tiles, partial words of a chunk
-    (700, 2100, 1004), (2100, 4100, 76), (40, 70, 30), (520, 300, 1001),        # 128- and 256-row tiles; staged k
+    (700, 2100, 1004), (40, 70, 30), (520, 300, 1001),                          # most 64x64 tiles; staged k
+    (1000, 2000, 1004), (1100, 1900, 508),                                      # auto: ragged 128x128, eight and four steps
+    (2100, 4100, 76), (2100, 4100, 132), (2100, 4100, 268), (2100, 4100, 396),  # auto: ragged 256x256, one to four steps
 ])
 def test_i8_products_of_every_size_are_exact(ctx, m, n, k):
     """The automatic choice and the small kernels against float64 dots (exact
