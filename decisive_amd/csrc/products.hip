@@ -2814,9 +2814,19 @@ int variant_count(const char *family) {
     return 0;
 }
 
+// The tuner's candidates: the first of each table. The tuner times one size and
+// keeps its winner for every size, so the tiles that are made for small grids
+// and win there only are left to the automatic rules: a tuner that took them
+// pinned 64x64p4 for the int8 products, 10 runs in 10 (8192 rows, K=N=4096:
+// 234 us against 128 by the rule), and small64x128, which is what pipe-auto runs at the
+// tuner's size, takes 3026 us against 1483 at 16384 rows, K=4096, N=14336.
 int tuned_count(const char *family) {
-    // the token scans and "auto" regroup the chunked scan's arithmetic
-    if (std::string(family) == "delta_scan") return 2;
+    const std::string f(family);
+    if (f == "delta_scan") return 2;  // the token scans and "auto" regroup the chunked scan's arithmetic
+    if (f == "gemm_w4a16") return 10;
+    if (f == "i8_gemm") return 11;
+    if (f == "grouped") return 14;
+    if (f == "mlp") return 6;
     return variant_count(family);
 }
 

@@ -555,7 +555,9 @@ int32_t dz_pplx_residency_info(dz_ctx *ctx, dz_pplx *model, char *json, size_t c
 
 /* Times the tile variants of every tuned kernel family within budget_ms and
  * keeps the fastest variant whose output is bitwise equal to the family's
- * reference variant and faster than 0.99x it. Families, in the reference's
+ * reference variant and faster than 0.99x it. A selection made at one size
+ * holds for all, so tiles made for small grids are no candidates (the
+ * reference variants pick them where they win). Families, in the reference's
  * stage order (checkpoint.rs:251-262): "delta_scan" (:328-421
  * select_delta_scan: 128 tokens of 32 value and 16 key heads; only the two
  * chunked scans, which keep the default's summation order, are candidates),

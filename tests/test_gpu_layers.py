@@ -345,6 +345,14 @@ def _tuner_checks(ctx):
     # the delta scan's candidates are the chunked scans only (select_delta_scan, checkpoint.rs:328-421)
     assert fams["delta_scan"]["candidates"] == ["chunked64", "chunked64-c32"]
     assert fams["delta_scan"]["shape"] == [128, 32, 16]
+    # the tiles for small grids are the automatic rules' alone: a selection holds for every size
+    small = {"gemm_w4a16": {"small32x32", "small32x64", "small64x64", "small64x128"}, "mlp": {"pipe64x64n4"},
+             "i8_gemm": {"rows", "64x64p4", "128x128p3w8"}, "grouped": {"pipe32x64w4g4", "pipe16x64w4g4"}}
+    for fam, names in small.items():
+        assert not names & set(fams[fam]["candidates"]), fam
+        for name in names:
+            ctx.select_variant(fam, name)  # selectable by name all the same
+        ctx.select_variant(fam, sel["selected"][fam])
     assert list(sel["selected"]) == list(TUNED)
     assert fams["norm"]["shape"][0] == 64 and fams["norm"]["shape"][2] == 2560
     again = ctx.tune(5000, cache=__import__("json").dumps(sel))
