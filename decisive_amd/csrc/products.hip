@@ -2929,8 +2929,13 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 //    waves; a grid too small for that is bound by the chain of steps of one
 //    block, so it takes four groups per step (half the barriers and twice the
 //    work between a load and its use; on fuller grids that is 2-5% slower) and
-//    the tile with the shortest step: 16x64 up to two and a half blocks per
-//    unit, else 32x64.
+//    the tile with the shortest step: 16x64 below two and a half blocks per
+//    unit, then 32x64; but of Q4 weights 32x128, two on a unit at most, once a
+//    fourth 32x64 block would come on some (us, 32x128w8g4 / 32x64w4g4, 32x64
+//    blocks per unit in brackets: N=2560, K=9216, 576 rows [2.8] 52.8 / 48.3,
+//    640 [3.1] 53.6 / 55.9, 800 [3.9] 58.8 / 61.4, affine 68.8 / 71.8; K=4096,
+//    640 rows 30.1 / 30.6; N=8192, K=2560, 192 rows [3.0] 20.2 / 18.5, 224
+//    [3.5] 21.5 / 22.0; Q8, N=2560, K=9216, 640 rows 69.0 / 67.9).
 // Measured there (us, 32x128w8g4 / 32x64w4g4 / 16x64w4g4 at 40, 128, 192 rows):
 // N=2560, K=9216 33.4 / 30.2 / 26.2, 35.5 / 32.8 / 28.8, 37.0 / 34.5 / 30.6;
 // N=2560, K=4096 19.1 / 17.2 / 15.4, 21.4 / 18.4 / 16.9, 21.4 / 19.9 / 18.0;
@@ -2951,7 +2956,8 @@ int grouped_pick(const Weight &w, int m, int variant) {
     const unsigned b64 = cdiv(m, 64) * tn;
     if (b64 >= 2 * cus && b64 % cus == 0) return 8;
     if (cdiv(m, 32) * tn >= 2 * cus) return 12;
-    return 2 * cdiv(m, 16) * cdiv(w.rows, 64) < 5 * cus ? 15 : 14;
+    if (2 * cdiv(m, 16) * cdiv(w.rows, 64) < 5 * cus) return 15;
+    return w.bits == 4 && cdiv(m, 32) * cdiv(w.rows, 64) > 3 * cus ? 9 : 14;
 }
 
 // Activation rows per block of a pipelined pick (0: not a pipelined kernel).

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from decisive_amd import rocm
-from gpu_util import bits_equal, dev, empty, host
+from gpu_util import bits_equal, dev, empty, host, launched
 
 pytestmark = pytest.mark.gpu
 
@@ -151,6 +151,31 @@ def test_grouped_four_group_tiles_give_the_one_wave_kernels_bits(ctx, bits, m, k
         ctx.select_variant("grouped", "pipe-auto")
     for name in out:
         assert bits_equal(out[name], out["wave16x16"]), name
+
+
+@pytest.mark.parametrize("bits,m,n,tile", [
+    (4, 208, 2560, "16, 64, 1, 4"), (4, 240, 2560, "16, 64, 1, 4"), (4, 241, 2560, "32, 64, 1, 4"),  # 2.5 16x64 blocks per unit
+    (4, 608, 2560, "32, 64, 1, 4"), (4, 640, 2560, "32, 128, 1, 8"), (4, 800, 2560, "32, 128, 1, 8"),  # three 32x64
+    (4, 192, 8192, "32, 64, 1, 4"), (4, 193, 8192, "32, 128, 1, 8"), (8, 640, 2560, "32, 64, 1, 4"),
+])
+def test_grouped_rule_takes_the_measured_tile(ctx, bits, m, n, tile):
+    """On both sides of the lines of the grouped rule for grids below two
+    32x128 blocks per unit (256 units): the tile that runs, with four groups
+    per step, and its bits."""
+    torch = pytest.importorskip("torch")
+    k = 192
+    rng = np.random.default_rng(m + n + bits)
+    w = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.05).astype(np.float32)), rocm.F32, n, k, bits, 64)
+    x = dev(rng.standard_normal((m, k)).astype(np.float32))
+    y, want = empty((m, n), torch.float32), empty((m, n), torch.float32)
+    got = launched(ctx, lambda: ctx.linear(w, x, rocm.F32, m, y, rocm.W4A8))
+    assert any(f"grouped_pipe_kernel<{bits}, {tile}, false, 4>" in g for g in got), got
+    try:
+        ctx.select_variant("grouped", "wave16x16")
+        ctx.linear(w, x, rocm.F32, m, want, rocm.W4A8)
+    finally:
+        ctx.select_variant("grouped", "pipe-auto")
+    assert bits_equal(host(ctx, y), host(ctx, want))
 
 
 @pytest.mark.parametrize("m,k,n", [(1, 64, 64), (3, 128, 64), (4, 192, 128), (63, 320, 64), (65, 1088, 192), (129, 576, 64)])
