@@ -1950,7 +1950,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void grouped_pipe_kernel(
     const int qd = lane / 16, j = lane % 16;
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
     int tm, tn;
-    xcd_tile(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    xcd_tile<BITS == 8>(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
     const int row0 = tm * BM, col0 = tn * BN;
     const int tiles = (n + 15) / 16, tile0 = col0 / 16, tvalid = min(TILES, tiles - tile0);
     const int rvalid = min(BM, m - row0);
@@ -2935,7 +2935,12 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 //    blocks per unit in brackets: N=2560, K=9216, 576 rows [2.8] 52.8 / 48.3,
 //    640 [3.1] 53.6 / 55.9, 800 [3.9] 58.8 / 61.4, affine 68.8 / 71.8; K=4096,
 //    640 rows 30.1 / 30.6; N=8192, K=2560, 192 rows [3.0] 20.2 / 18.5, 224
-//    [3.5] 21.5 / 22.0; Q8, N=2560, K=9216, 640 rows 69.0 / 67.9).
+//    [3.5] 21.5 / 22.0; Q8, N=2560, K=9216, 640 rows 69.0 / 67.9). Of Q8
+//    weights 16x64 up to two blocks per unit (us, 32x128w8g4 / 32x64w4g4 /
+//    16x64w4g4, 16x64 blocks per unit in brackets: N=4160, K=9216, 97 rows
+//    [1.8] 35.8 / 32.1 / 27.2, 129 rows [2.3] 37.4 / 34.1 / 42.7; N=2560,
+//    K=4096, 177 rows [1.9] 20.4 / 18.1 / 16.6, 209 rows [2.2] 21.2 / 19.9 /
+//    20.5).
 // Measured there (us, 32x128w8g4 / 32x64w4g4 / 16x64w4g4 at 40, 128, 192 rows):
 // N=2560, K=9216 33.4 / 30.2 / 26.2, 35.5 / 32.8 / 28.8, 37.0 / 34.5 / 30.6;
 // N=2560, K=4096 19.1 / 17.2 / 15.4, 21.4 / 18.4 / 16.9, 21.4 / 19.9 / 18.0;
@@ -2956,7 +2961,8 @@ int grouped_pick(const Weight &w, int m, int variant) {
     const unsigned b64 = cdiv(m, 64) * tn;
     if (b64 >= 2 * cus && b64 % cus == 0) return 8;
     if (cdiv(m, 32) * tn >= 2 * cus) return 12;
-    if (2 * cdiv(m, 16) * cdiv(w.rows, 64) < 5 * cus) return 15;
+    const unsigned b16 = cdiv(m, 16) * cdiv(w.rows, 64);
+    if (w.bits == 4 ? 2 * b16 < 5 * cus : b16 <= 2 * cus) return 15;
     return w.bits == 4 && cdiv(m, 32) * cdiv(w.rows, 64) > 3 * cus ? 9 : 14;
 }
 
