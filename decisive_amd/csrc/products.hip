@@ -2926,21 +2926,24 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 //    the rest; 1280 32x64 blocks put five on each). So 128x128 side by side
 //    when their grid gives every unit four blocks, else 64x128 on 8 waves
 //    when its grid is two or more whole blocks per unit, else 32x64 on 4
-//    waves; a grid too small for that is bound by the chain of steps of one
-//    block, so it takes four groups per step (half the barriers and twice the
-//    work between a load and its use; on fuller grids that is 2-5% slower) and
-//    the tile with the shortest step: 16x64 below two and a half blocks per
-//    unit, then 32x64; but of Q4 weights 32x128, two on a unit at most, once a
-//    fourth 32x64 block would come on some (us, 32x128w8g4 / 32x64w4g4, 32x64
-//    blocks per unit in brackets: N=2560, K=9216, 576 rows [2.8] 52.8 / 48.3,
-//    640 [3.1] 53.6 / 55.9, 800 [3.9] 58.8 / 61.4, affine 68.8 / 71.8; K=4096,
-//    640 rows 30.1 / 30.6; N=8192, K=2560, 192 rows [3.0] 20.2 / 18.5, 224
-//    [3.5] 21.5 / 22.0; Q8, N=2560, K=9216, 640 rows 69.0 / 67.9). Of Q8
-//    weights 16x64 up to two blocks per unit (us, 32x128w8g4 / 32x64w4g4 /
-//    16x64w4g4, 16x64 blocks per unit in brackets: N=4160, K=9216, 97 rows
-//    [1.8] 35.8 / 32.1 / 27.2, 129 rows [2.3] 37.4 / 34.1 / 42.7; N=2560,
-//    K=4096, 177 rows [1.9] 20.4 / 18.1 / 16.6, 209 rows [2.2] 21.2 / 19.9 /
-//    20.5).
+//    waves;
+//  - a grid of less than two 32x128 blocks per unit is bound by the chain of
+//    steps of one block, so it takes four groups per step (half the barriers and
+//    twice the work between a load and its use; on fuller grids that is 2-5%
+//    slower) and the tile with the shortest step while the units hold its
+//    blocks. In us, 32x128w8g4 / 32x64w4g4 / 16x64w4g4:
+//    16x64, for Q8 up to two blocks per unit (N=4160, K=9216, 97 rows, 1.8 per
+//    unit, 35.8 / 32.1 / 27.2; 129 rows, 2.3, 37.4 / 34.1 / 42.7), for Q4 below
+//    two and a half (N=2560, K=4096, 225 rows, 2.3, 19.6 / 19.0 / 18.9; N=1183,
+//    K=2328, 454 rows, 2.2, 17.0 / 16.6 / 15.8), or two and a quarter on up to
+//    five tile rows whose grid is not whole rounds of the XCDs (N=9520, K=8616, 53
+//    rows, 2.3, 32.0 / 31.1 / 34.4; N=8000, K=9216, 70 rows, 2.4, 33.9 / 32.9 /
+//    35.1);
+//    then 32x64, or for Q4 32x128 once a fourth 32x64 block would come on some
+//    units (N=2560, K=9216, 576 rows, 2.8 per unit, 52.8 / 48.3; 640 rows, 3.1,
+//    53.6 / 55.9; 800 rows 58.8 / 61.4, affine 68.8 / 71.8, Q8 73.3 / 73.0), of
+//    rows that are stored a value at a time only at K from 2048 (N=3869, K=896,
+//    503 rows 15.8 / 15.1; N=2082, K=8992, 903 rows 63.8 / 67.0).
 // Measured there (us, 32x128w8g4 / 32x64w4g4 / 16x64w4g4 at 40, 128, 192 rows):
 // N=2560, K=9216 33.4 / 30.2 / 26.2, 35.5 / 32.8 / 28.8, 37.0 / 34.5 / 30.6;
 // N=2560, K=4096 19.1 / 17.2 / 15.4, 21.4 / 18.4 / 16.9, 21.4 / 19.9 / 18.0;
@@ -2962,8 +2965,10 @@ int grouped_pick(const Weight &w, int m, int variant) {
     if (b64 >= 2 * cus && b64 % cus == 0) return 8;
     if (cdiv(m, 32) * tn >= 2 * cus) return 12;
     const unsigned b16 = cdiv(m, 16) * cdiv(w.rows, 64);
-    if (w.bits == 4 ? 2 * b16 < 5 * cus : b16 <= 2 * cus) return 15;
-    return w.bits == 4 && cdiv(m, 32) * cdiv(w.rows, 64) > 3 * cus ? 9 : 14;
+    const bool q4_15 = 2 * b16 < 5 * cus && (b16 % 8 == 0 || 4 * b16 < 9 * cus || m > 80);
+    if (w.bits == 4 ? q4_15 : b16 <= 2 * cus) return 15;
+    const bool q4_9 = (w.rows % 4 == 0 || w.groups >= 32) && cdiv(m, 32) * cdiv(w.rows, 64) > 3 * cus;
+    return w.bits == 4 && q4_9 ? 9 : 14;
 }
 
 // Activation rows per block of a pipelined pick (0: not a pipelined kernel).

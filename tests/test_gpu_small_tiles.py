@@ -157,6 +157,8 @@ def test_grouped_four_group_tiles_give_the_one_wave_kernels_bits(ctx, bits, m, k
     (4, 208, 2560, "16, 64, 1, 4"), (4, 240, 2560, "16, 64, 1, 4"), (4, 241, 2560, "32, 64, 1, 4"),  # 2.5 16x64 blocks per unit
     (4, 608, 2560, "32, 64, 1, 4"), (4, 640, 2560, "32, 128, 1, 8"), (4, 800, 2560, "32, 128, 1, 8"),  # three 32x64
     (4, 192, 8192, "32, 64, 1, 4"), (4, 193, 8192, "32, 128, 1, 8"), (8, 640, 2560, "32, 64, 1, 4"),
+    (4, 48, 9520, "16, 64, 1, 4"), (4, 53, 9520, "32, 64, 1, 4"), (4, 454, 1183, "16, 64, 1, 4"), (4, 125, 4672, "16, 64, 1, 4"),
+    (4, 503, 3869, "32, 64, 1, 4"),  # stored a value at a time, few groups
     (8, 97, 4160, "16, 64, 1, 4"), (8, 113, 4160, "32, 64, 1, 4"), (8, 192, 2560, "16, 64, 1, 4"),   # Q8: two 16x64 per unit;
     (8, 208, 2560, "32, 64, 1, 4"), (8, 300, 4005, "32, 64, 1, 4"),                                # some grids not whole rounds
 ])
