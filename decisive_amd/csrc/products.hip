@@ -3039,7 +3039,12 @@ bool launch_grouped(const Weight &w, const int8_t *q, const float *sx, int m, fl
 // 392 / 385; N=1024, 229 rows 39.8 / 28.1; K=4096, N=14336, 229 rows 79.5 /
 // 76.2, 4096 rows 916 / 901. Up to three rows the one-wave blocks, which read no
 // empty rows (1 row, one-wave / 64-row: N=1024 23.9 / 26.6, K=4096, N=14336 36.4
-// / 38.9; at 4 rows 26.9 / 26.4 and 43.8 / 38.6).
+// / 38.9; at 4 rows 26.9 / 26.4 and 43.8 / 38.6), and also where a product is of
+// up to five groups and a unit gets one of them at most, so that a block is
+// mostly its prologue (N=512, 64 rows, K=64 8.1 / 9.2, K=192 9.3 / 10.1, K=320
+// 10.7 / 11.1, K=384 11.5 / 11.4; N=1024, K=192, 800 rows, 3.1 per unit, 12.1 /
+// 10.4), at three groups one and a quarter (N=1024, 300 rows 10.1 / 10.3) and at
+// one two and a half (N=3072, 200 rows 9.1 / 9.4, 300 rows 9.9 / 9.4).
 // All variants are word-exact with the unfused composition.
 void launch_mlp_requant(const Weight &gate, const Weight &up, const int8_t *q, const float *sx,
                         int m, int8_t *qo, float *so, const int *bad, int variant, hipStream_t s) {
@@ -3048,7 +3053,10 @@ void launch_mlp_requant(const Weight &gate, const Weight &up, const int8_t *q, c
     const bool fits = (size_t)256 * gate.groups * 64 < ((size_t)1 << 31) &&
                       (size_t)4 * gate.kblocks() * 1024 < ((size_t)1 << 31) && ((uintptr_t)qo & 3) == 0 &&
                       gate.rows % 4 == 0;
-    const int pick = variant != 0 ? variant : m < 4 ? 3 : 6;
+    const unsigned cus = (unsigned)device_cus(), b16 = cdiv(m, 16) * tn;
+    const bool short_blocks =
+        gate.groups <= 5 && 4 * b16 <= (gate.groups == 1 ? 10 : gate.groups <= 3 ? 5 : 4) * cus;
+    const int pick = variant != 0 ? variant : m < 4 || short_blocks ? 3 : 6;
     const auto launch = [&](auto kernel, int bm, int waves) {
         hipLaunchKernelGGL(kernel, dim3(cdiv(m, bm) * tn), dim3(waves * 64), 0, s, gate.codes, gate.scales, up.codes,
                            up.scales, q, sx, m, gate.rows, gate.groups, gate.kblocks(), qo, so, bad);

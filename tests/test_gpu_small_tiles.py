@@ -205,3 +205,24 @@ def test_mlp_64_row_blocks_give_the_one_wave_kernels_bits(ctx, m, k, n):
         ctx.select_variant("mlp", "pipe-auto")
     for name in out:
         assert np.array_equal(out[name][0], out["wave16x64"][0]) and bits_equal(out[name][1], out["wave16x64"][1]), name
+
+
+@pytest.mark.parametrize("m,k,n,small", [
+    (3, 640, 64, True), (4, 384, 64, False),                                    # rows
+    (64, 320, 1024, True), (64, 384, 1024, False),                              # five groups
+    (256, 320, 1024, True), (257, 320, 1024, False),                            # one block per unit
+    (320, 192, 1024, True), (321, 192, 1024, False), (320, 256, 1024, False),   # one and a quarter, up to three groups
+    (640, 64, 1024, True), (641, 64, 1024, False),                              # two and a half, at one group
+])
+def test_mlp_rule_takes_the_measured_blocks(ctx, m, k, n, small):
+    """On both sides of the lines between the one-wave and the 64-row blocks
+    (256 units): the kernel that runs."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(m + n + k)
+    gate, up = (ctx.quantize(dev((rng.standard_normal((n, k)) * 0.05).astype(np.float32)), rocm.F32, n, k, 4, 64)
+                for _ in range(2))
+    x = dev(rng.standard_normal((m, k)).astype(np.float32))
+    q, s = empty((m, n), torch.int8), empty((m, n // 64), torch.float32)
+    got = launched(ctx, lambda: ctx.mlp_requant(gate, up, x, m, q, s))
+    want = "mlp_requant_kernel" if small else "mlp_pipe_kernel<64, 4, 1>"
+    assert any(want in g for g in got), got
