@@ -2708,7 +2708,8 @@ bool w4a16_pipe_launch(const Weight &w, const half_t *x, int m, void *y, const h
 // through registers. All give the same bits (same f16 dequantization, one MFMA per
 // 32-k run in k order). Where k % 128 != 0 the pipelined kernel has 256x256
 // and 128x128 tiles; its other forms, and panels past 32-bit offsets, fall back
-// to 256x128w2x2 (K=1688, N=1063: 45 us at 1024 rows and 47 at 2048).
+// to 256x128w2x2 (K=1688, N=1063: 45 us at 1024 rows and 47 at 2048). There
+// "auto" takes 128x128w2x2 for short products of rows that are not whole vectors.
 template <int EPI>
 void gemm_dispatch(const Weight &w, const half_t *x, int m, void *y, const half_t *res, int variant,
                    hipStream_t s) {
@@ -2719,6 +2720,16 @@ void gemm_dispatch(const Weight &w, const half_t *x, int m, void *y, const half_
             const unsigned cus = (unsigned)device_cus();
             const unsigned tm = cdiv(m, 256), tn = cdiv(w.rows, 256);
             if (w.cols % 128 != 0) {  // the ragged form: 256x256 tiles from one per unit, else 128x128
+                // Rows that are stored a value at a time cost the pipelined tiles, whose lanes hold four
+                // columns, more than the staged ones, whose lanes hold one: with the stores a good part of
+                // a short product, the staged 128x128 (us, pipelined / staged: N=12001, K=328, 2000 rows 73.5 /
+                // 38.7; N=6981, K=800, 800 rows 30.8 / 25.4; N=6009, 2000 rows, K=1072 55.8 / 47.8, f16 49.8 /
+                // 45.9, K=1688 70.5 / 69.1, f16 64.8 / 66.8; N=4122, K=1144, 531 rows 19.9 / 20.7). With
+                // GELU 47.9 / 50.2 and with a residual 67.8 / 73.2 at K=1072.
+                if (EPI <= 1 && w.rows % 4 != 0 && w.cols < 1088) {
+                    gemm_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s);
+                    return;
+                }
                 if (tm * tn >= cus ? w4a16_pipe_launch<256, 256, 2, 4, EPI>(w, x, m, y, res, s)
                                    : w4a16_pipe_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s))
                     return;

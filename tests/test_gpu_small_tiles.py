@@ -49,6 +49,27 @@ def test_w4a16_small_tiles_give_the_staged_kernels_bits(ctx, group, m, k, n):
         ctx.select_variant("gemm_w4a16", "pipe-auto")
 
 
+@pytest.mark.parametrize("m,k,n,kernel,tile", [
+    (700, 1080, 4001, "gemm_w4a16_kernel", (128, 128)), (700, 1096, 4001, "w4a16_pipe_kernel", (128, 128)),    # short products
+    (700, 1080, 4004, "w4a16_pipe_kernel", (128, 128)), (700, 1024, 4001, "w4a16_pipe_kernel", (128, 128)),    # whole vectors, k-blocks
+    (300, 1080, 4001, "w4a16_small_kernel", (64, 128)), (4100, 200, 4099, "gemm_w4a16_kernel", (128, 128)),    # small tiles first
+])
+def test_w4a16_rule_at_ragged_k_takes_the_measured_kernel(ctx, m, k, n, kernel, tile):
+    """On both sides of the lines of the rule where k is not whole blocks (256
+    units): the kernel that runs, for f32 and plain f16 outputs, and no staged
+    one through the other epilogues."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(k)
+    w = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.02).astype(np.float32)), rocm.F32, n, k, 4, 32)
+    x, y, h = dev(rng.standard_normal((m, k)).astype(np.float16)), empty((m, n), torch.float32), empty((m, n), torch.float16)
+    forms = ["{}<{}, {},".format(kernel, *tile), "{}ILi{}ELi{}E".format(kernel, *tile)]  # demangled or not
+    for run in (lambda: ctx.linear(w, x, rocm.F16, m, y, rocm.W4A16), lambda: ctx.linear_f16(w, x, m, h, rocm.EPI_NONE)):
+        got = launched(ctx, run)
+        assert any(f in g for g in got for f in forms), got
+    got = launched(ctx, lambda: ctx.linear_f16(w, x, m, h, rocm.EPI_GELU))
+    assert not any("gemm_w4a16_kernel" in g for g in got), got
+
+
 @pytest.mark.parametrize("k", [1000, 4096])
 def test_w4a16_rows_do_not_see_each_other(ctx, k):
     """A row of infinities beside finite ones: the chunks a partial block loads
