@@ -2719,7 +2719,10 @@ void gemm_dispatch(const Weight &w, const half_t *x, int m, void *y, const half_
         case 0: {
             const unsigned cus = (unsigned)device_cus();
             const unsigned tm = cdiv(m, 256), tn = cdiv(w.rows, 256);
-            if (w.cols % 128 != 0) {  // the ragged form: 256x256 tiles from one per unit, else 128x128
+            if (w.cols % 128 != 0) {
+                // the ragged form: 256x256 tiles at one per unit and from one and a quarter, where the second
+                // round is not mostly empty, else 128x128 (us, 256x256 / 128x128, K=4720: 1331 rows, N=10824, 1.01
+                // per unit, 214 / 156; 2048 rows, N=10240, 1.25, 227 / 204; N=11264, 1.38, 229 / 232)
                 // Rows that are stored a value at a time cost the pipelined tiles, whose lanes hold four
                 // columns, more than the staged ones, whose lanes hold one: with the stores a good part of
                 // a short product, the staged 128x128 (us, pipelined / staged: N=12001, K=328, 2000 rows 73.5 /
@@ -2730,8 +2733,9 @@ void gemm_dispatch(const Weight &w, const half_t *x, int m, void *y, const half_
                     gemm_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s);
                     return;
                 }
-                if (tm * tn >= cus ? w4a16_pipe_launch<256, 256, 2, 4, EPI>(w, x, m, y, res, s)
-                                   : w4a16_pipe_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s))
+                const bool large = tm * tn == cus || 4 * tm * tn > 5 * cus;
+                if (large ? w4a16_pipe_launch<256, 256, 2, 4, EPI>(w, x, m, y, res, s)
+                          : w4a16_pipe_launch<128, 128, 2, 2, EPI>(w, x, m, y, res, s))
                     return;
                 break;
             }

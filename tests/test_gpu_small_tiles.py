@@ -52,6 +52,8 @@ def test_w4a16_small_tiles_give_the_staged_kernels_bits(ctx, group, m, k, n):
 @pytest.mark.parametrize("m,k,n,kernel,tile", [
     (700, 1080, 4001, "gemm_w4a16_kernel", (128, 128)), (700, 1096, 4001, "w4a16_pipe_kernel", (128, 128)),    # short products
     (700, 1080, 4004, "w4a16_pipe_kernel", (128, 128)), (700, 1024, 4001, "w4a16_pipe_kernel", (128, 128)),    # whole vectors, k-blocks
+    (4096, 136, 4096, "w4a16_pipe_kernel", (256, 256)), (4097, 136, 4096, "w4a16_pipe_kernel", (128, 128)),    # one 256x256 per unit
+    (5120, 136, 4096, "w4a16_pipe_kernel", (128, 128)), (5121, 136, 4096, "w4a16_pipe_kernel", (256, 256)),    # one and a quarter
     (300, 1080, 4001, "w4a16_small_kernel", (64, 128)), (4100, 200, 4099, "gemm_w4a16_kernel", (128, 128)),    # small tiles first
 ])
 def test_w4a16_rule_at_ragged_k_takes_the_measured_kernel(ctx, m, k, n, kernel, tile):
