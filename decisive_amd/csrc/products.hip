@@ -3183,9 +3183,15 @@ bool i8_stream_launch(const int8_t *a, const float *sa, int m, const int8_t *b, 
 //    rows 37.5 / 27.8 / 33.5 / 45.6, 2048 rows 68.7 / 52.1 / 45.6 / 52.2);
 //  - 256x256 (4096 rows 125.9 / 94.2 / 81.8 / 70.9).
 // Where k % 16 != 0 the ragged forms of 64x64, 128x128 and 256x256 (also in
-// 256x128's place) take k % 4 == 0, and any other k is staged: on 64x64 tiles up to three 128x128 blocks
-// for every two units (K=1000, N=1063, 300 rows 16.1 against 32.6), 128x128
-// beyond. Every variant computes exact int32 dots, so all are bitwise equal;
+// 256x128's place) take k % 4 == 0. Any other k is staged, as the Q4 weight is:
+// on 64x64 tiles (K=1000, N=1063, 300 rows 16.1 against 32.6 on 128x128) up to
+// the four blocks that a unit holds, three past k = 8192, where the 128x128
+// tiles' fewer bytes count, four and a half at k <= 2048 and six, one and a half 128x128 blocks,
+// at k <= 1024, and for Q4, which is half the bytes, up to five, six at k <= 2048 (us, 64x64 / 128x128:
+// K=1002, 4.6 per unit 37.3 / 44.0; K=2049, 4.5, 48.5 / 47.5, 5.2, 61.3 / 51.2; K=4610, 4.0, 77.7 / 80.1,
+// 4.25, 88.2 / 82.5; K=6145, 5.2, 157.6 / 112.0; K=9218, 3.2, 147.9 / 141.2; Q4
+// K=4096, 4.4 per unit 0.83 of 128x128's time, 5.1 1.02, K=1000, 5.9 0.82).
+// Every variant computes exact int32 dots, so all are bitwise equal;
 // when a pipelined variant cannot take a shape, the register-staged 128x128 runs.
 template <bool Q4B>
 void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, const float *sb, int n,
@@ -3216,7 +3222,8 @@ void i8_gemm_dispatch(const int8_t *a, const float *sa, int m, const int8_t *b, 
             default: break;
         }
     }
-    if (variant == 0 && 2 * grid(128, 128) <= 3 * cus) variant = 6;
+    const size_t most64 = Q4B ? (k <= 2048 ? 12 : 10) : k <= 1024 ? 12 : k <= 2048 ? 9 : k <= 8192 ? 8 : 6;  // per two units
+    if (variant == 0 && 2 * grid(64, 64) <= most64 * cus) variant = 6;
     switch (variant) {
         case 5:
             hipLaunchKernelGGL((i8_gemm_kernel<256, 128, 2, 2, Q4B>), dim3(cdiv(n, 128), cdiv(m, 256)), dim3(256), 0,

@@ -661,6 +661,22 @@ def test_i8_variant_names_run_their_kernels(ctx):
         ctx.select_variant("i8_gemm", "auto")
 
 
+@pytest.mark.parametrize("m,n,k,tile", [
+    (2048, 2048, 4097, 64), (2048, 2112, 4097, 128),                             # four 64x64 blocks per unit
+    (1536, 2048, 8194, 64), (1536, 2112, 8194, 128),                             # three past k = 8192
+    (2048, 2304, 2047, 64), (2048, 2368, 2047, 128), (2048, 2304, 2049, 128),    # four and a half at k <= 2048
+    (2048, 3072, 1023, 64), (2048, 3136, 1023, 128), (2048, 3072, 1025, 128),    # six at k <= 1024
+])
+def test_i8_staged_rule_takes_the_measured_tile(ctx, m, n, k, tile):
+    """At a k that is not whole words, on both sides of the lines between the
+    staged 64x64 and 128x128 tiles (256 units): the kernel that runs."""
+    torch = pytest.importorskip("torch")
+    a, b = (torch.randint(-127, 128, s, dtype=torch.int8, device="cuda") for s in ((m, k), (n, k)))
+    y = empty((m, n), torch.int32)
+    got = launched(ctx, lambda: ctx.i8_gemm(a, None, m, b, None, n, k, y, raw=True))
+    assert any(f"i8_gemm_kernel<{tile}, {tile}," in g for g in got), got
+
+
 @pytest.mark.parametrize("m,n,k", [[1, 1, 4], [77, 45, 100], [130, 260, 4100], [256, 512, 4096], [513, 257, 80]])
 def test_i8_gemm_fused_silu(ctx, oracle, m, n, k):
     """webgpu/int8.rs:226-230 fused mode against the oracle: bit for bit but
