@@ -312,15 +312,28 @@ template <class F, int... I>
 __device__ __forceinline__ void each_index(F f, std::integer_sequence<int, I...>) {
     (f(std::integral_constant<int, I>{}), ...);
 }
-// acc = fma(lane L of a's 16-lane row, x, acc). As asm, since the compiler leaves
-// the broadcast a move of its own; the operand `a` comes from LDS and passes
-// dpp_ready first (a DPP read needs two wait states after a VALU write).
-template <int L>
-__device__ __forceinline__ float fma_row_lane(float a, float x, float acc) {
-    asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(a), "v"(x), "n"(L));
-    return acc;
+// s[l % 4] = fma(lane l of a's 16-lane row, x[l], s[l % 4]) for the whole quads of
+// l < N in turn, and what is left of them onto s[0]. As asm, since the compiler leaves
+// the broadcasts moves of their own, and as one block: a DPP read needs two wait
+// states after a VALU write of its operand, which the compiler does not see to inside
+// asm, so the wait stands in the block and no register copy of `a` can come after it.
+#define DZ_FMAC_LANE(part, x, l) "v_fmac_f32_dpp %" #part ", %4, %" #x " row_newbcast:" #l " row_mask:0xf bank_mask:0xf\n\t"
+#define DZ_FMAC_STEP(part, x, l)                                    \
+    ".if " #l " < (%21 & 28)\n\t" DZ_FMAC_LANE(part, x, l)          \
+    ".elseif " #l " < %21\n\t" DZ_FMAC_LANE(0, x, l) ".endif\n\t"
+template <int N>
+__device__ __forceinline__ void fma_row(float a, const float (&x)[16], float (&s)[4]) {
+    asm("s_nop 1\n\t"
+        DZ_FMAC_STEP(0, 5, 0) DZ_FMAC_STEP(1, 6, 1) DZ_FMAC_STEP(2, 7, 2) DZ_FMAC_STEP(3, 8, 3)
+        DZ_FMAC_STEP(0, 9, 4) DZ_FMAC_STEP(1, 10, 5) DZ_FMAC_STEP(2, 11, 6) DZ_FMAC_STEP(3, 12, 7)
+        DZ_FMAC_STEP(0, 13, 8) DZ_FMAC_STEP(1, 14, 9) DZ_FMAC_STEP(2, 15, 10) DZ_FMAC_STEP(3, 16, 11)
+        DZ_FMAC_STEP(0, 17, 12) DZ_FMAC_STEP(1, 18, 13) DZ_FMAC_STEP(2, 19, 14) DZ_FMAC_STEP(3, 20, 15)
+        : "+&v"(s[0]), "+&v"(s[1]), "+&v"(s[2]), "+&v"(s[3])
+        : "v"(a), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]),
+          "v"(x[9]), "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]), "n"(N));
 }
-__device__ __forceinline__ void dpp_ready(float &a) { asm volatile("s_nop 1" : "+v"(a)); }
+#undef DZ_FMAC_STEP
+#undef DZ_FMAC_LANE
 
 __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__restrict__ qhat,
                                                                const float *__restrict__ khat,
@@ -495,24 +508,12 @@ __global__ __launch_bounds__(256) void delta_chunk_prep_kernel(const float *__re
 #pragma unroll
             for (int l = 0; l < 16; l++) xc[l] = xcol[(16 * c + l) * kChunkRow];
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                float a = ab[r * 16];
-                dpp_ready(a);
-                each_index([&](auto l) { s[r][l % 4] = fma_row_lane<l>(a, xc[l], s[r][l % 4]); },
-                           std::make_integer_sequence<int, 16>{});
-            }
+            for (int r = 0; r < 16; r++) fma_row<16>(ab[r * 16], xc, s[r]);
         }
         each_index(
             [&](auto row) {
                 constexpr int r = decltype(row)::value;
-                float a = ab[r * 16];
-                dpp_ready(a);
-                each_index(
-                    [&](auto l) {
-                        constexpr int part = l < (r & ~3) ? l % 4 : 0;
-                        if constexpr (l < r) s[r][part] = fma_row_lane<l>(a, x[l], s[r][part]);
-                    },
-                    std::make_integer_sequence<int, 16>{});
+                if constexpr (r > 0) fma_row<r>(ab[r * 16], x, s[r]);
                 if (r > 0 || b > 0) x[r] -= (s[r][0] + s[r][1]) + (s[r][2] + s[r][3]);
             },
             std::make_integer_sequence<int, 16>{});
