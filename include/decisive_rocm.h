@@ -585,7 +585,9 @@ int32_t dz_tune(dz_ctx *ctx, uint32_t budget_ms, const char *cache_in, char *cac
  *                 stream8 for 2..8 rows over eight or more tiles per compute unit)
  *   "gemm_w4a16"  pipe-auto, 256x256p2w8, 128x128p2w4, 128x256p2w8, 256x128w2x2,
  *                 128x128w2x2, 128x64w2x2, 256x256p2w8-persist, 256x192p2w8-persist,
- *                 256x128p2w8
+ *                 256x128p2w8, small32x32, small32x64, small64x64, small64x128
+ *                 (the tiles pipe-auto takes first, where their grid is at most
+ *                 one block per compute unit)
  *   "i8_gemm"     auto, 256x256p4k64w8, 256x128p3w8, 256x128p3, 128x128w2x2,
  *                 256x128w2x2, 64x64w2x2, 256x256p2w8-stream, 256x256p2w8-stream-mid,
  *                 256x128k64p2-stream2 (the "-stream" forms are persistent: one
@@ -599,9 +601,10 @@ int32_t dz_tune(dz_ctx *ctx, uint32_t budget_ms, const char *cache_in, char *cac
  *                 pipe32x128w8g4, pipe64x128w8g4 (g4: four 64-groups per
  *                 pipeline step instead of two), fewrow16 (the few-row kernel,
  *                 16 rows per block row, over the A8 codes), pipe32x64w4,
- *                 pipe64x64w8
+ *                 pipe64x64w8, pipe32x64w4g4, pipe16x64w4g4
  *   "mlp"         pipe-auto, pipe256x64w8, pipe128x64w4, wave16x64, pipe256x64n2,
- *                 pipe128x64n2
+ *                 pipe128x64n2, pipe64x64n4 (what pipe-auto runs but for the
+ *                 smallest calls, which take wave16x64)
  *   "delta_scan"  chunked64, chunked64-c32, recurrent, recurrent-rolled,
  *                 auto (the decider's gated delta rule. The default runs the
  *                 rule by 64-token chunks with 16 state columns per block;

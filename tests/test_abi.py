@@ -2,9 +2,13 @@
 
 No compute call is made here (no GPU in the CPU suite)."""
 import ctypes
+import re
 import subprocess
+from pathlib import Path
 
 from decisive_amd import rocm
+
+ROOT = Path(__file__).resolve().parent.parent
 
 
 def test_header_declares_entry_points():
@@ -41,3 +45,16 @@ def test_init_without_gpu_reports_gpu_unavailable():
     rc = rocm.load().dz_init(0, ctypes.byref(h))
     assert rocm.STATUS_NAMES[rc] in ("GPU_UNAVAILABLE", "MISSING_GPU_FEATURE")
     assert h.value is None
+
+
+def test_header_lists_every_selectable_variant():
+    """The variant tables of products.hip against dz_select_variant's list, in order."""
+    tables = dict(gemv="kGemvNames", gemm_w4a16="kGemmNames", i8_gemm="kI8Names", grouped="kGroupedNames",
+                  mlp="kMlpNames", delta_scan="kDeltaNames", norm="kNormNames")
+    source = (ROOT / "decisive_amd" / "csrc" / "products.hip").read_text()
+    header = (ROOT / "include" / "decisive_rocm.h").read_text().rsplit("int32_t dz_select_variant", 1)[0]
+    for family, table in tables.items():
+        names = re.findall(r'"([^"]+)"', re.search(table + r"\[\] = \{(.*?)\};", source, re.S).group(1))
+        listed = re.search(r'\n \*   "' + family + r'" (.*?)(?=\n \*   "|\*/)', header, re.S).group(1)
+        words = re.findall(r"[\w-]+", listed)
+        assert names and not set(names) - set(words), (family, set(names) - set(words))
