@@ -384,7 +384,8 @@ def test_tuned_grouped_and_mlp_variants_agree_on_real_inputs(ctx, oracle):
     x = dev(rng.standard_normal((m, k)).astype(np.float32))
     outs = []
     for v in ("pipe-auto", "pipe256x128w8", "wave16x16", "pipe128x128w4", "pipe64x128w2", "pipe128x128m8",
-              "pipe128x128n8", "pipe32x128w8", "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16", "pipe32x64w4", "pipe64x64w8"):
+              "pipe128x128n8", "pipe32x128w8", "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16", "pipe32x64w4",
+              "pipe64x64w8", "pipe32x64w4g4", "pipe16x64w4g4"):
         ctx.select_variant("grouped", v)
         y = empty((m, n), torch.float32)
         ctx.linear(w, x, rocm.F32, m, y, rocm.W4A8)
@@ -398,7 +399,8 @@ def test_tuned_grouped_and_mlp_variants_agree_on_real_inputs(ctx, oracle):
     u = ctx.quantize(dev((rng.standard_normal((n, k)) * 0.02).astype(np.float32)), rocm.F32, n, k, 4, 64)
     x = dev(rng.standard_normal((m, k)).astype(np.float32))
     outs = []
-    for v in ("pipe-auto", "pipe256x64w8", "pipe128x64w4", "wave16x64", "pipe256x64n2", "pipe128x64n2"):
+    for v in ("pipe-auto", "pipe256x64w8", "pipe128x64w4", "wave16x64", "pipe256x64n2", "pipe128x64n2",
+              "pipe64x64n4"):
         ctx.select_variant("mlp", v)
         q, s = empty((m, n), torch.int8), empty((m, n // 64), torch.float32)
         ctx.mlp_requant(g, u, x, m, q, s)

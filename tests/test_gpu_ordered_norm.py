@@ -52,6 +52,26 @@ def test_readout_norm_adds_in_row_order(ctx, oracle, kind, d):
         assert bits_equal(got[r], oracle.project(packed, 8, d, x[r], n)), r
 
 
+@pytest.mark.parametrize("d,at", [(64, 0), (576, 300), (2560, 2559), (8192, 4100)])
+@pytest.mark.parametrize("bad", [np.nan, -np.nan, np.inf, -np.inf])
+def test_readout_norm_reports_nonfinite_rows(ctx, oracle, bad, d, at):
+    """A NaN or infinite term takes the sum out of the last binade: the row's
+    norm is not finite, as the serial loop's is not, and the next call is
+    unaffected."""
+    torch = pytest.importorskip("torch")
+    packed = oracle.pack_g64(oracle.f32_to_bf16(np.full((3, d), 0.01, np.float32)), 3, d, 8)
+    w = ctx.upload(packed, rocm.Q8_G64_F32, 3, d)
+    norm, logits = np.zeros(d, np.float32), empty((4, 3), torch.float32)
+    clean = _rows("normal", 4, d)
+    rows = clean.copy()
+    rows[2, at] = bad
+    with pytest.raises(rocm.DzError, match="nonfinite readout activation"):
+        ctx.readout(w, dev(norm), dev(rows), 4, EPS, logits)
+    ctx.readout(w, dev(norm), dev(clean), 4, EPS, logits)
+    want = oracle.project(packed, 8, d, oracle.rmsnorm(clean, norm, EPS, zero_centered=True)[2], 3)
+    assert bits_equal(host(ctx, logits)[2], want)
+
+
 @pytest.mark.parametrize("hidden", [192, 1024, 1088, 3072, 3136, 4096, 4160])
 def test_quantizing_norm_of_every_row_width(ctx, oracle, hidden):
     """The codes' block holds 1024, 3072, 4096 or 8192 columns; each gives the

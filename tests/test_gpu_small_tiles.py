@@ -5,6 +5,8 @@ import pytest
 
 from decisive_amd import rocm
 from gpu_util import bits_equal, dev, empty, host, launched
+from tests import pplx_model
+from tests.test_gpu_pplx import SMALL
 
 pytestmark = pytest.mark.gpu
 
@@ -172,6 +174,29 @@ def test_grouped_four_group_tiles_give_the_one_wave_kernels_bits(ctx, bits, m, k
             assert (out[name][m * n:] == -7.0).all(), name
     finally:
         ctx.select_variant("grouped", "pipe-auto")
+    for name in out:
+        assert bits_equal(out[name], out["wave16x16"]), name
+
+
+@pytest.mark.parametrize("layer,n", [(1, 17), (1, 37), (1, 130), (3, 77)])
+def test_four_group_tiles_add_the_residual_in_their_store(ctx, oracle, layer, n):
+    """out_proj, o_proj and down_proj onto the hidden rows, on the 32x64 and
+    16x64 tiles and by the separate add of the one-wave kernel."""
+    pytest.importorskip("torch")
+    model = pplx_model.random_model(oracle, SMALL, seed=4)
+    p = pplx_model.load(ctx, rocm, model)
+    h = np.random.default_rng(n).standard_normal((n, SMALL["hidden"])).astype(np.float32)
+    out = {}
+    for name in ("wave16x16", "pipe32x64w4", "pipe32x64w4g4", "pipe16x64w4g4"):
+        hd = dev(h)
+        ctx.select_variant("grouped", name)
+        try:
+            p.layer(layer, hd, n)
+        finally:
+            ctx.select_variant("grouped", "pipe-auto")
+        out[name] = host(ctx, hd)
+    p.close()
+    assert np.isfinite(out["wave16x16"]).all()
     for name in out:
         assert bits_equal(out[name], out["wave16x16"]), name
 
