@@ -1,8 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the MI355X quantized matrix-product path.
 
-Headline (BASELINE.json metric, configuration 2): the bandwidth-bound Q4 GEMV,
-W4A16, M = 1 row of f16 activations, K = N = 4096, g32/f16 weights.
+Headline: the bandwidth-bound Q4 GEMV, W4A16, M = 1 row of f16 activations, K = N = 4096, g32/f16 weights.
 A step is one pass of the activations through WEIGHT_COPIES distinct Q4
 [4096 x 4096] weights (one GEMV launch each, replayed as one HIP graph), so
 the 256 MB Infinity Cache cannot serve repeated weights and the number is an
@@ -175,7 +174,7 @@ def cpu_baseline(seconds: float = 8.0) -> dict:
 
 
 def encoder_cpu_baseline(seconds: float = 8.0) -> dict:
-    """Config 3's encoder layer on the host cores, for one 1024-token sequence:
+    """The encoder's layer on the host cores, for one 1024-token sequence:
     the four projections by the reference's CPU W4A8 algorithm (C restatement
     of int8.rs:229-585, AVX2 rows<4,Q4>, threaded), attention by numpy float32
     matrix products (the reference's CPU attention is an sgemm), LayerNorm and
@@ -247,7 +246,7 @@ def encoder_cpu_baseline(seconds: float = 8.0) -> dict:
 
 
 def gemv_lines(torch, ctx, rocm, weights, stream) -> dict:
-    """Config 2 at M = 4 and 8 (W4A16) and the bit-exact W4A8 GEMV at M = 1."""
+    """The headline GEMV at M = 4 and 8 (W4A16) and the bit-exact W4A8 GEMV at M = 1."""
     out = {}
     for m in (4, 8):
         x = torch.randn((m, K_DIM), generator=torch.Generator(device="cuda").manual_seed(0), device="cuda").half()
@@ -323,7 +322,7 @@ def w4a8_line(torch, ctx, rocm, stream) -> dict:
 
 
 def encoder_line(torch, ctx, rocm, stream) -> dict:
-    """Config 3: the encoder forward, 24 x (1024, 16x64, 4096), batch 8 x 1024
+    """The encoder forward, 24 x (1024, 16x64, 4096), batch 8 x 1024
     tokens, random Q4 g32 weights."""
     cfg = rocm.EncoderConfig(layers=24, hidden=1024, heads=16, head_dim=64, ffn=4096, vocab=32000, ln_eps=1e-5)
     enc = ctx.encoder_random(cfg, 1)
@@ -340,7 +339,7 @@ def encoder_line(torch, ctx, rocm, stream) -> dict:
 
 
 def int8_line(torch, ctx, stream) -> dict:
-    """Config 4: the per-row int8 GEMM at M=8192, K=N=4096 (f32 out), the
+    """The per-row int8 GEMM at M=8192, K=N=4096 (f32 out), the
     vendor library on the same codes, and the same launch on all-zero codes."""
     m, n, k = 8192, 4096, 4096
     a = torch.randn((m, k), generator=torch.Generator(device="cuda").manual_seed(0), device="cuda")
@@ -387,7 +386,7 @@ def int8_line(torch, ctx, stream) -> dict:
 
 def secondary(torch, ctx, rocm, stream, cpu=True) -> dict:
     out = {"int8_gemm_m8192_k4096_n4096": int8_line(torch, ctx, stream)}
-    # config 5: Q4 prefill M=16384 K=4096 N=14336
+    # Q4 prefill M=16384 K=4096 N=14336
     m, k, n = 16384, 4096, 14336
     wf = torch.randn((n, k), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 0.02
     torch.cuda.synchronize()
@@ -417,7 +416,7 @@ def secondary(torch, ctx, rocm, stream, cpu=True) -> dict:
         "note": "dz_linear_f16: f32 accumulation, each output rounded once to f16"}
     w.free()
     del x, y
-    # the reference's own numerics (bit-exact W4A8, int8.rs fold order) at the config 5 shape:
+    # the reference's own numerics (bit-exact W4A8, int8.rs fold order) at the same shape:
     # f32 activations quantized to A8 on device, then the grouped product
     wf = torch.randn((n, k), generator=torch.Generator(device="cuda").manual_seed(1), device="cuda") * 0.02
     torch.cuda.synchronize()

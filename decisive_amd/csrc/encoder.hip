@@ -1,4 +1,4 @@
-// encoder.hip -- the encoder forward of BASELINE configuration 3 on the
+// encoder.hip -- the embedding encoder's forward on the
 // quantized-product kernels.
 //
 // Layer order follows the reference's post-LayerNorm encoder

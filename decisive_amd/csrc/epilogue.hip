@@ -365,7 +365,7 @@ __global__ __launch_bounds__(W * 64, 4) void attention_kernel(const half_t *__re
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
     const int q4 = lane / 16, j = lane % 16;
     // blocks in (query block, head, batch) order, a contiguous share per XCD
-    // (xcd_unit): the 8 sequences of 1024 tokens of configuration 3 each run on
+    // (xcd_unit): 8 sequences of 1024 tokens each run on
     // the XCD whose product blocks wrote their qkv rows
     constexpr int QUERIES = W * kAttnQB * 16;  // per block
     constexpr int ROWS = kAttnKeys / W;        // K and V rows each wave copies per step

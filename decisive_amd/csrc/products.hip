@@ -1304,7 +1304,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void i8_gemm_pipe_kernel(const int8_
     // into it are issued in SUBS slices, one before each substep's MFMAs.
     // With two stages they are issued in two slices, before the first two
     // substeps, so that the last of them has most of the step to land
-    // (config 4, alternated on one box: 123.3-123.9 us against 126.9-128.1
+    // (8192 rows, K=N=4096, alternated on one box: 123.3-123.9 us against 126.9-128.1
     // with all of them before the first substep and 130.0-131.5 with four
     // slices; three slices 1.2% slower than two; with three stages the four
     // slices pay)
@@ -1659,7 +1659,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, 2) void i8_gemm_stream_kernel(const 
 // barrier; the one compute body reads whichever stage is current. Needs
 // k % 128 == 0, or RAGGED (k % 8 == 0): the chunks of a partial last block,
 // which hold the next row's values, are then cleared in LDS before that step
-// (a form of its own: the test for it costs config 5's product 0.5%).
+// (a form of its own: the test for it costs 16384 rows, K=4096, N=14336 0.5%).
 // Codes become f16 exactly as in gemm_w4a16_kernel (exact code times the f16
 // scale, rounded once), and each output accumulates one
 // v_mfma_f32_16x16x32_f16 per 32-k run in k order, so both kernels give the
@@ -1723,8 +1723,8 @@ __global__ __launch_bounds__(WGM *WGN * 64) void w4a16_pipe_kernel(
     const uint32_t xlane = (uint32_t)(q * k * 2);
     const int cx = j ^ q;
     // the next step's loads are spread over the first groups: over two, each
-    // load has longer to land than over four (config 5: 1.526-1.529 against
-    // 1.540-1.543 ms with f16 output, 1.545-1.556 against 1.572-1.582 with f32;
+    // load has longer to land than over four (16384 rows, K=4096, N=14336:
+    // 1.526-1.529 against 1.540-1.543 ms with f16 output, 1.545-1.556 against 1.572-1.582 with f32;
     // the encoder 6.78-6.83 against 6.86-6.93 ms; all at once: in between)
     constexpr int DMA_GROUPS = 2;
     constexpr int DMA_N = XPW + WPW;
@@ -2231,12 +2231,13 @@ __global__ __launch_bounds__(WGM *WGN * 64) void grouped_pipe_kernel(
 // of each weight): a weight fragment is unpacked once for four row blocks
 // rather than two, and the row maximum takes one exchange through LDS between
 // the pair. BM = 64 with WN = 4 (wave tile 64 rows x 16 columns of each weight)
-// is what the products run: it is bound by the fold's VALU work (three
-// operations per output, group and weight) and, on small grids, by the
-// dependent steps of one wave, so it takes few enough registers for four waves
-// per SIMD (126; reading a step's scales or codes at once takes 130 and the
-// fourth wave) and orders dots before folds (fold_step). Two more load stages
-// changed nothing.
+// is what the products run. Counters at K=2560, N=9216: the fold's VALU work
+// (three operations per output, group and weight) issues for 0.54 of the time at
+// 1024 rows and 0.35 at 229, the MFMA pipe is busy 0.24 and 0.18, and the rest are
+// the waits at a step's barrier and the dependent steps of a wave. So it takes few
+// enough registers for four waves per SIMD (126; reading a step's scales or codes
+// at once takes 130 and the fourth wave) and orders dots before folds
+// (fold_step). Two more load stages changed nothing.
 template <int BM, int WN = 1, int WM = BM / (32 * WN)>
 __global__ __launch_bounds__(WM *WN * 64) void mlp_pipe_kernel(
     const uint8_t *__restrict__ gcodes, const uint8_t *__restrict__ gscales, const uint8_t *__restrict__ ucodes,
@@ -2891,10 +2892,6 @@ void launch_grouped_records(const Weight &w, const uint32_t *records, int m, flo
     gv_launch<2, false>(w, records, nullptr, m, 8, y, nullptr, nullptr, s);
 }
 
-// Variant 1 is grouped_pipe_kernel (256x128 tiles, 8 waves), variant 2 the
-// one-wave-per-16x16-tile grouped_kernel, variant 0 ("auto") the first when
-// its grid covers at least half the compute units and the second otherwise.
-// All fold in the reference order, so all give the same bits.
 // The pipelined grouped kernels address a BM-row activation panel and a
 // weight tile column with 32-bit byte offsets.
 bool grouped_pipe_fits(const Weight &w, int bm) {

@@ -2,8 +2,8 @@
 // (src/inference/mod.rs:140-154) over the C ABI of libdecisive_rocm.so.
 //
 // It takes the place of `impl Backend for pplx_flash::Model` (the native CPU
-// backend, src/inference/adapters.rs:168-194) for the Pplx-style encoder of
-// BASELINE configuration 3:
+// backend, src/inference/adapters.rs:168-194) for the Pplx-style
+// encoder (24 layers of 1024, 16 heads of 64, FFN 4096):
 //   Parameters = PplxParameters (maxSequenceTokens, default 1024, 0 rejected)
 //   CacheState = EmbeddingCache (packed Q4 g64/f32 embedding rows by token id)
 //   capabilities = {model "pplx-flash", backend "rocm", caches ["embedding"], tuning "auto"}

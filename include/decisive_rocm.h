@@ -241,7 +241,7 @@ int32_t dz_linear_noalloc(dz_ctx *ctx, const dz_weight *w, const void *x_dev, in
  * two weights with the same cols. */
 int32_t dz_linear_pair(dz_ctx *ctx, const dz_weight *a, const dz_weight *b, const float *x_dev,
                        size_t m, float *ya_dev, float *yb_dev, int32_t mode);
-/* The prefill form of DZ_W4A16 (the encoder's
+/* The prefill form of DZ_W4A16 (16384 rows at 4096 x 14336; the encoder's
  * projections): f16 activations x_dev [m x cols(w)] (16-byte aligned) ->
  * f16 y_dev [m x rows(w)]: the products accumulate in f32 as dz_linear's
  * DZ_W4A16 does, and each output is rounded to f16 once, after the epilogue:
@@ -344,7 +344,7 @@ int32_t dz_mean_rows(dz_ctx *ctx, const void *x_dev, int32_t dtype, size_t batch
 int32_t dz_attention(dz_ctx *ctx, const void *qkv_dev, void *out_dev, size_t batch, size_t seq,
                      size_t heads, size_t dh, float scale);
 
-/* ---- encoder forward -------------------------------- */
+/* ---- encoder forward --------------------------------------------------------- */
 
 typedef struct dz_encoder_config {
     int32_t layers;     /* 24   */

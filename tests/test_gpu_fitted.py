@@ -14,7 +14,7 @@ from decisive_amd import rocm
 from tests.gpu_util import bits_equal, cosine, dev, empty, host
 
 pytestmark = pytest.mark.gpu
-MAX_ABS = 1e-2  # north_star tolerance for f16/f32 GEMM outputs
+MAX_ABS = 1e-2  # tolerance for f16/f32 GEMM outputs
 MIN_COS = 0.9999
 GROUPED_VARIANTS = ("pipe256x128w8", "wave16x16", "pipe128x128w4", "pipe64x128w2", "pipe128x128m8",
                     "pipe128x128n8", "pipe32x128w8", "pipe64x128w8", "pipe32x128w8g4", "pipe64x128w8g4", "fewrow16", "pipe32x64w4",
@@ -78,7 +78,7 @@ def test_scaled_fit_grouped_products_bit_exact(ctx, oracle, m, k, n):
 
 @pytest.mark.parametrize("m,k,n", [(1, 4096, 512), (8, 1024, 300), (64, 512, 256)])
 def test_scaled_fit_w4a16_vs_closed_form(ctx, oracle, m, k, n):
-    """W4A16 takes MSE-fitted weights: the f64 closed form within north_star."""
+    """W4A16 takes MSE-fitted weights: the f64 closed form within tolerance."""
     torch = pytest.importorskip("torch")
     _, codes, scales, _ = fitted(oracle, n, k, "mse", n + k)
     w = upload(ctx, oracle, codes, scales, None, n, k, rocm.FIT_SCALED)

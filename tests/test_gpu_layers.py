@@ -10,7 +10,7 @@ from decisive_amd import rocm
 from tests.gpu_util import bits_equal, cosine, dev, empty, host
 
 pytestmark = pytest.mark.gpu
-MAX_ABS = 1e-2  # north_star tolerance for f16/f32 GEMM and layer outputs
+MAX_ABS = 1e-2  # tolerance for f16/f32 GEMM and layer outputs
 MIN_COS = 0.9999
 
 
@@ -267,7 +267,7 @@ def test_encoder_bits_do_not_depend_on_the_gemm_variant(ctx):
 
 
 def test_config3_width_encoder_matches_composition(ctx, oracle):
-    """Config 3's layer shape (hidden 1024, 16 heads of 64, FFN 4096, vocab
+    """The embedding encoder's layer shape (hidden 1024, 16 heads of 64, FFN 4096, vocab
     32000) at 2 layers over two 1024-token sequences: the kernels that run at
     full size (wave-per-row LayerNorm at 1024, 16-head attention over 1024
     keys, the 256x256 and 128x256 pipelined GEMM tiles with their GELU and

@@ -50,7 +50,7 @@ def act(ctx, p, name, shape, dtype):
     return host(ctx, t).copy()
 
 
-def north_star(got, want, what):
+def within_tolerance(got, want, what):
     err = float(np.abs(got.astype(np.float64) - want).max())
     cos = float(cosine(got, want))
     print(f"{what}: max |d| {err:.3e} (largest |value| {float(np.abs(want).max()):.3f}), cosine {cos:.9f}")
@@ -121,11 +121,11 @@ def test_delta_mixer_ops_against_the_oracle_on_the_gpus_inputs(ctx, oracle, real
         assert bits_equal(got, product(oracle, model, pre + f"linear_attn.{name}.weight", nc, ns)), name
     conv = act(ctx, p, "conv", (N, cw), torch.float32)
     taps = v[pre + "linear_attn.conv1d.weight"].reshape(cw, 4).T.copy()
-    north_star(conv, oracle.conv_silu(qkv, taps), "conv + SiLU")
+    within_tolerance(conv, oracle.conv_silu(qkv, taps), "conv + SiLU")
     heads = act(ctx, p, "heads", (lh, N, LD), torch.float32)
     decay = np.exp(v[pre + "linear_attn.A_log"]).astype(np.float32)
     want = oracle.delta_scan(conv, lh, lk, LD, a, b, decay, v[pre + "linear_attn.dt_bias"])
-    north_star(heads, want, "delta prep + scan")
+    within_tolerance(heads, want, "delta prep + scan")
     gc = act(ctx, p, "gate_codes", (N, lv), torch.int8)
     gs = act(ctx, p, "gate_scales", (N, lv // 64), torch.float32)
     gated = oracle.delta_gate(heads, v[pre + "linear_attn.norm.weight"], z)
@@ -171,13 +171,13 @@ def test_attention_mixer_ops_against_the_oracle_on_the_gpus_inputs(ctx, oracle, 
     query = act(ctx, p, "query", (nq, ah * AD), torch.float32)
     want_q = oracle.rope(pplx_model._head_norm(oracle, q_part, ah, v[pre + "self_attn.q_norm.weight"]), ah, AD, pos,
                          freq)
-    north_star(query, want_q, "query head norm + rotary")
+    within_tolerance(query, want_q, "query head norm + rotary")
     key = act(ctx, p, "key", (N, akv * AD), torch.float32)
     want_k = oracle.rope(pplx_model._head_norm(oracle, key_raw, akv, v[pre + "self_attn.k_norm.weight"]), akv, AD,
                          np.arange(N), freq)
-    north_star(key, want_k, "key head norm + rotary")
+    within_tolerance(key, want_k, "key head norm + rotary")
     heads = act(ctx, p, "heads", (ah, nq, AD), torch.float32)
-    north_star(heads, oracle.attention_gqa(query, key, value, ah, akv, AD, 1.0 / 16.0), "GQA attention")
+    within_tolerance(heads, oracle.attention_gqa(query, key, value, ah, akv, AD, 1.0 / 16.0), "GQA attention")
     gated = oracle.attention_gate(heads, z)
     if mk is None:
         gc = act(ctx, p, "gate_codes", (nq, ah * AD), torch.int8)
@@ -186,7 +186,7 @@ def test_attention_mixer_ops_against_the_oracle_on_the_gpus_inputs(ctx, oracle, 
         proj = product(oracle, model, pre + "self_attn.o_proj.weight", gc, gs)
     else:
         g = act(ctx, p, "gate", (nq, ah * AD), torch.float32)
-        north_star(g, gated, "attention gate")
+        within_tolerance(g, gated, "attention gate")
         gq, gsq = oracle.act_quantize(g, nq, ah * AD, 8)  # the product quantizes its f32 input
         proj = product(oracle, model, pre + "self_attn.o_proj.weight", gq, gsq)
     rows = h if mk is None else h[mk]

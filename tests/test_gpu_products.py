@@ -15,7 +15,7 @@ from tests.gpu_util import bits_equal, cosine, dev, empty, host, launched
 
 pytestmark = pytest.mark.gpu
 GOLDEN = json.loads((Path(__file__).parent / "golden" / "reference_vectors.json").read_text())
-MAX_ABS = 1e-2  # north_star tolerance for f16/f32 GEMM outputs
+MAX_ABS = 1e-2  # tolerance for f16/f32 GEMM outputs
 MIN_COS = 0.9999
 
 
@@ -120,7 +120,7 @@ def test_kernel_check_cases_vs_project(ctx, oracle, case, bits):
 
 
 def test_config1_q4_linear_bit_exact(ctx, oracle):
-    """BASELINE config 1: x N(0,1) [128 x 1024] seed 0, W N(0,0.02) [1024 x 1024]
+    """x N(0,1) [128 x 1024] seed 0, W N(0,0.02) [1024 x 1024]
     seed 1, through the reference's g64 quantizer (BF16 input)."""
     torch = pytest.importorskip("torch")
     m = k = n = 1024
@@ -292,7 +292,7 @@ def test_fused_mlp_requant_equals_unfused(ctx, oracle):
 
 @pytest.mark.parametrize("m", [1, 4, 8])
 def test_config2_gemv_vs_closed_form(ctx, oracle, m):
-    """BASELINE config 2: f16 x N(0,1) seed 0, K = N = 4096, W N(0,0.02) seed 1, g32/f16."""
+    """f16 x N(0,1) seed 0, K = N = 4096, W N(0,0.02) seed 1, g32/f16."""
     torch = pytest.importorskip("torch")
     k = n = 4096
     x = np.random.default_rng(0).standard_normal((m, k)).astype(np.float32)
@@ -584,7 +584,7 @@ def test_w4a16_column_split_matches_register_kernel(ctx, oracle, n):
 
 
 def test_config5_prefill_rows_vs_fp32(ctx, oracle):
-    """BASELINE config 5 at full size (M=16384, K=4096, N=14336); a row sample is
+    """The Q4 prefill at full size (M=16384, K=4096, N=14336); a row sample is
     checked against an fp32 product of the dequantized weights."""
     torch = pytest.importorskip("torch")
     m, k, n = 16384, 4096, 14336
@@ -708,7 +708,7 @@ def test_i8_gemm_fused_silu(ctx, oracle, m, n, k):
 
 
 def test_config4_int8_full_size(ctx, oracle):
-    """BASELINE config 4: W f32 [4096 x 4096] N(0,0.02) per-channel, A f32
+    """W f32 [4096 x 4096] N(0,0.02) per-channel, A f32
     [8192 x 4096] N(0,1) per-token; quantized on the GPU (bit-exact with the
     oracle) and the i32 accumulators bit-exact on a row sample."""
     torch = pytest.importorskip("torch")
