@@ -1950,7 +1950,7 @@ __global__ __launch_bounds__(WGM *WGN * 64) void grouped_pipe_kernel(
     const int qd = lane / 16, j = lane % 16;
     const int tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
     int tm, tn;
-    xcd_tile<BITS == 8>(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn);
+    xcd_tile(blockIdx.x, gridDim.x, tiles_m, tiles_n, tm, tn, BITS == 8 && groups > 4);
     const int row0 = tm * BM, col0 = tn * BN;
     const int tiles = (n + 15) / 16, tile0 = col0 / 16, tvalid = min(TILES, tiles - tile0);
     const int rvalid = min(BM, m - row0);

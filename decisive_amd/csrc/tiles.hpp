@@ -14,18 +14,19 @@ inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 // so tile ids are taken in XCD-major order and grouped GROUP_M tile-rows at a
 // time, keeping the blocks that share an XCD's L2 on neighbouring tiles. A grid
 // that is not whole rounds of the XCDs is taken in block order, where every L2
-// reads all of the weight, or, with ANY and more than a block per compute unit,
-// in XCD order too: the grouped Q8 products are bound by that (us, 16x64 tiles,
-// N=4160, K=9216: 81 rows 37.9 in block order, 26.7 so; 97 rows 39.7 and 27.0).
+// reads all of the weight, or, with `any` and more than a block per compute unit,
+// in XCD order too: the grouped Q8 products past four groups are bound by that (us,
+// 16x64 tiles, N=4160, K=9216: 81 rows 37.9 in block order, 26.7 so; 97 rows 39.7 and
+// 27.0; 1282 rows, N=7992, K=512 34.4 and 28.8, but K=256 21.7 and 22.6, K=64 18.8 and 19.8).
 // The others, whose weights are half as large or whose stores weigh more, lose
 // by it (grouped Q4, 503 rows, K=896, N=3869 15.3 and 16.1; W4A16, 596 rows,
 // K=9360, N=6927 144 and 149; MLP, 264 rows, K=512, N=3520 13.2 and 13.7).
-template <bool ANY = false>
-__device__ __forceinline__ void xcd_tile(int bid, int nblocks, int tiles_m, int tiles_n, int &tm, int &tn) {
+__device__ __forceinline__ void xcd_tile(int bid, int nblocks, int tiles_m, int tiles_n, int &tm, int &tn,
+                                         bool any = false) {
     constexpr int XCDS = 8, GROUP_M = 4;
     int linear = bid;
     // XCD x has the blocks x, x + 8, ...: nblocks / 8 of them, and one more below the remainder
-    if (ANY && nblocks > 32 * XCDS)
+    if (any && nblocks > 32 * XCDS)
         linear = (bid % XCDS) * (nblocks / XCDS) + min(bid % XCDS, nblocks % XCDS) + bid / XCDS;
     else if (nblocks % XCDS == 0) linear = (bid % XCDS) * (nblocks / XCDS) + bid / XCDS;
     const int per_group = GROUP_M * tiles_n;
