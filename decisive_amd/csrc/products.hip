@@ -2953,7 +2953,8 @@ bool grouped_pipe_launch(const Weight &w, const int8_t *q, const float *sx, int 
 //    35.1), but past one and a half not for Q4 of up to 128 columns on such a grid
 //    at K below 2048, where the rows' bytes count and one 32x128 tile holds a row
 //    (N=128, K=896, 3538 rows, 1.7, 14.6 / 15.4 / 15.0; 5000 rows, 2.4, 16.5 /
-//    18.2 / 18.3; K=2048, 3538 rows 22.6 / 22.3 / 21.5);
+//    18.2 / 18.3; K=2048, 3538 rows 22.6 / 22.3 / 21.5), nor past two for such Q8 at
+//    K up to 256 (N=128, K=256, 7565 rows, 3.7, 11.1 / 11.8 / 13.1);
 //    then 32x64, or for Q4 32x128 once a fourth 32x64 block would come on some
 //    units (N=2560, K=9216, 576 rows, 2.8 per unit, 52.8 / 48.3; 640 rows, 3.1,
 //    53.6 / 55.9; 800 rows 58.8 / 61.4, affine 68.8 / 71.8, Q8 73.3 / 73.0), of
@@ -2980,7 +2981,8 @@ int grouped_pick(const Weight &w, int m, int variant) {
     if (b64 >= 2 * cus && b64 % cus == 0) return 8;
     if (cdiv(m, 32) * tn >= 2 * cus) return 12;
     const unsigned b16 = cdiv(m, 16) * cdiv(w.rows, 64);
-    if (w.bits == 4 && tn == 1 && b16 % 8 != 0 && 2 * b16 > 3 * cus && w.groups < 32) return 9;
+    const bool narrow = w.bits == 4 ? b16 % 8 != 0 && 2 * b16 > 3 * cus && w.groups < 32 : b16 > 2 * cus && w.groups <= 4;
+    if (tn == 1 && narrow) return 9;
     const bool q4_15 = 2 * b16 < 5 * cus && (b16 % 8 == 0 || 4 * b16 < 9 * cus || m > 80);
     if (w.bits == 4 ? q4_15 : b16 <= 2 * cus) return 15;
     const bool q4_9 = (w.rows % 4 == 0 || w.groups >= 32) && cdiv(m, 32) * cdiv(w.rows, 64) > 3 * cus;

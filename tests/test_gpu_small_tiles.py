@@ -208,6 +208,7 @@ def test_four_group_tiles_add_the_residual_in_their_store(ctx, oracle, layer, n)
     (4, 48, 9520, "16, 64, 1, 4"), (4, 53, 9520, "32, 64, 1, 4"), (4, 454, 1183, "16, 64, 1, 4"), (4, 125, 4672, "16, 64, 1, 4"),
     (4, 503, 3869, "32, 64, 1, 4"),  # stored a value at a time, few groups
     (4, 3538, 128, "32, 128, 1, 8"), (4, 3000, 128, "16, 64, 1, 4"), (4, 2600, 128, "16, 64, 1, 4"),  # one column of 32x128
+    (8, 4097, 128, "32, 128, 1, 8"), (8, 4096, 128, "16, 64, 1, 4"), (8, 4097, 129, "32, 64, 1, 4"),
     (8, 97, 4160, "16, 64, 1, 4"), (8, 113, 4160, "32, 64, 1, 4"), (8, 192, 2560, "16, 64, 1, 4"),   # Q8: two 16x64 per unit;
     (8, 208, 2560, "32, 64, 1, 4"), (8, 300, 4005, "32, 64, 1, 4"),                                # some grids not whole rounds
 ])
